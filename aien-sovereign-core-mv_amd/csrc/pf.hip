@@ -95,19 +95,31 @@ __global__ __launch_bounds__(256) void k_pf_quant(const PfQuantArgs a) {
 }
 
 // ------------------------------------------------------------------ grouped W8A8 GEMM
-// Workgroup = (tile of up to 64 activation rows of one expert, column span); wavefront w takes
-// two 16-row A tiles of the expert's row-major e4m3 weights: PLAIN, output columns
-// 128 x + 32 w .. +32; SWIGLU, gate rows j0 .. j0 + 16 and up rows I + j0 .. with j0 = 64 x + 16 w
-// (their act columns). The tile's activation rows (gathered through the row index) are staged per
-// 128-column k-block in LDS (rows padded to 144 bytes: the 16 rows a read instruction touches sit
-// on distinct banks) and shared by the four wavefronts. Per k-block, the e4m3 products run on the
-// matrix cores with the activation block scale as the B operand's E8M0 scale (a power of two, so
-// the products stay exact) and the f32 block sum is multiplied by the weight block scale into the
-// accumulator. Two k-block sets take turns on one straight path (the loads of one in flight while
-// the other is staged and multiplied); a set past the last k-block reloads the last one and
-// contributes with weight scale 0.
+// Workgroup = 64 RW weight rows (PLAIN: output columns 64 RW x ..; SWIGLU: gate rows 32 RW x .. and
+// the up rows of the same act columns) x one tile of up to 64 activation rows, RW x 2 wavefronts of
+// 64 weight rows x half of the activation rows each. RW 2 (three workgroups a CU) is the general
+// form. The paired form (RW 4, PLAIN) also takes two consecutive tiles of one expert at once; the
+// second tile's workgroup then leaves.
+//
+// What bounds it is the traffic into the CUs (about 20 bytes a clock each, L2 included) and, for
+// small tiles, the weights from HBM. So a load instruction of a wavefront reads 8 rows x one whole
+// 128-byte line (operand-shaped loads, 16 rows x 64 bytes, left the streams a third slower), rows
+// past the tile's count repeat its last row (an L1 hit), and XCDs own ranges of tiles or spans.
+// Both operands go through LDS, one 128-column k-block at a time: a thread loads 16-byte pieces in
+// registers two k-blocks ahead, writes them to the buffer that the previous step read, and one
+// barrier per k-block hands it over. Piece c of row r sits at slot c ^ (r % 8) of the row, so the
+// 16 rows that a matrix-core operand read touches fall on distinct banks without padding. Per
+// k-block, the e4m3 products run with the activation block scale as the B operand's E8M0 scale (a
+// power of two, so the products stay exact) and the f32 block sum is multiplied by the weight block
+// scale into the accumulator.
+//
+// Measured (launch times; the form with the weights loaded straight into operand registers and one
+// 64 x 128 tile per workgroup before): q|k|v 5120 x 2048 at 512 rows 31 -> 24 us, 4096 rows 170 ->
+// 93 us; o 2048 x 4096 at 4096 rows 135 -> 57 us; 128 experts at 2000 tokens gate|up 299 -> 151 us,
+// down 162 -> 110 us; at 100 tokens 108 -> 76 and 61 -> 38 us.
 struct PfGemmArgs {
-    uint32_t n = 0, k = 0, layout = 0;
+    uint32_t n = 0, k = 0, layout = 0, ntiles = 0;
+    uint32_t by_cols = 0;  // an XCD takes a range of column spans (else a range of tiles)
     const PfTile *tiles = nullptr;
     const uint32_t *rowidx = nullptr;  // nullptr: output row r reads activation row r
     const uint8_t *xq = nullptr;       // [rows][k] e4m3
@@ -115,123 +127,198 @@ struct PfGemmArgs {
     void *y = nullptr;                 // PLAIN f32 [rows][n]; SWIGLU bf16 [rows][n / 2]
 };
 
-constexpr uint32_t kPfRow = 144;  // staged bytes per activation row
+constexpr uint32_t kPfMaxKb = 32768 / 128;
 
-struct PfSet {
-    u32x4 a[2][2];  // A tiles: lane (g, n): row n, bytes 16 g .. +16 and 64 + 16 g .. +16
-    u32x4 b[2];     // staged activation bytes: thread t: row t / 4, bytes 32 (t % 4) .. +32
-    float bs;       // thread t < 64: the block scale of row t
+template <int AROWS, int BROWS>
+struct PfLds {
+    uint8_t a[2][AROWS * 128];
+    uint8_t b[2][BROWS * 128];
+    int sb[2][BROWS];        // E8M0 exponents of the rows' block scales
+    float ws[2][kPfMaxKb];   // weight block scales of the two halves of the weight rows
 };
 
-template <int LAYOUT>
-__global__ __launch_bounds__(256) void k_pf_qgemm(const PfGemmArgs a) {
-    __shared__ __align__(16) uint8_t xb[2][kPfBm * kPfRow];
-    __shared__ float xsb[2][kPfBm];
+// the two 16-byte pieces of a lane's operand: row n of the 16 rows at `t`, pieces g and g + 4
+__device__ __forceinline__ i32x8 pf_frag(const uint8_t *t, uint32_t off) {
+    const u32x4 lo = *reinterpret_cast<const u32x4 *>(t + off), hi = *reinterpret_cast<const u32x4 *>(t + (off ^ 64));
+    return i32x8{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+}
+
+// RW x 2 wavefronts: 64 RW weight rows; BT: 16-row B tiles per wavefront (2: one tile of the table,
+// 4: two)
+template <int LAYOUT, int RW, int BT, class Lds>
+__device__ __forceinline__ void pf_qgemm_wg(const PfGemmArgs &a, Lds &L, uint64_t w_va, uint64_t s_va, uint32_t x,
+                                            uint32_t row0, uint32_t cnt) {
     const uint32_t tid = threadIdx.x, lane = lane_id(), w = tid >> 6, g = lane >> 4, n = lane & 15;
-    const PfTile *tp = a.tiles + blockIdx.y;
-    const cu32 *tw = as_const_u32(tp);
+    const uint32_t KB = a.k / 128, wr = w >> 1, wc = w & 1;
+    // first weight row of the two halves
+    constexpr bool kSwiglu = LAYOUT == kPfLayoutSwiglu;
+    constexpr uint32_t kThreads = 128 * RW, kHalf = 32 * RW, kPass = 16 * RW, NB = 2 * BT / RW;
+    const uint32_t h0 = kSwiglu ? kHalf * x : 2 * kHalf * x;
+    const uint32_t h1 = kSwiglu ? a.n / 2 + h0 : h0 + kHalf;
+    const uint8_t *wt = reinterpret_cast<const uint8_t *>(w_va);
+    const float *ws = reinterpret_cast<const float *>(s_va);
+    for (uint32_t i = tid; i < KB; i += kThreads) {
+        L.ws[0][i] = *as_global_f32(ws + (size_t)(h0 >> 7) * KB + i);
+        L.ws[1][i] = *as_global_f32(ws + (size_t)(h1 >> 7) * KB + i);
+    }
+    // staging: thread t takes pieces of rows t / 8 + kPass i, slot t % 8
+    const uint32_t sr = tid >> 3, piece = ((tid & 7) ^ (sr & 7)) * 16;
+    const uint32_t woff = sr * a.k + piece;
+    const uint8_t *xp[NB];
+    const float *xsp[NB];
+#pragma unroll
+    for (uint32_t i = 0; i < NB; ++i) {
+        const uint32_t r = row0 + min(sr + kPass * i, cnt - 1), src = a.rowidx ? *as_global_u32(a.rowidx + r) : r;
+        xp[i] = a.xq + (size_t)src * a.k + piece;
+        xsp[i] = a.xs + (size_t)src * KB;
+    }
+    struct Set {
+        u32x4 a[4], b[NB];
+        float s[NB];
+    };
+    auto load = [&](Set &S, uint32_t kb) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S.a[i] = *as_global(wt + ((size_t)((i < 2 ? h0 : h1) + kPass * (i & 1)) * a.k + 128 * kb) + woff);
+#pragma unroll
+        for (uint32_t i = 0; i < NB; ++i) S.b[i] = *as_global(xp[i] + 128 * kb);
+#pragma unroll
+        for (uint32_t i = 0; i < NB; ++i) S.s[i] = *as_global_f32(xsp[i] + kb);
+    };
+    auto stage = [&](const Set &S, int u) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4 *>(L.a[u] + 16 * tid + 16 * kThreads * i) = S.a[i];
+#pragma unroll
+        for (uint32_t i = 0; i < NB; ++i) *reinterpret_cast<u32x4 *>(L.b[u] + 16 * tid + 16 * kThreads * i) = S.b[i];
+        if ((tid & 7) == 0)
+#pragma unroll
+            for (uint32_t i = 0; i < NB; ++i) L.sb[u][sr + kPass * i] = e8m0_of(S.s[i]);
+    };
+    f32x4 tot[4][BT];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < BT; ++j) tot[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint32_t off = n * 128 + ((g ^ (n & 7)) << 4);
+    // 16-row A tiles of the wavefront: PLAIN 4 wr .. 4 wr + 3; SWIGLU gate tiles 2 wr, 2 wr + 1 and
+    // the up tiles of the same columns
+    const uint32_t at0 = kSwiglu ? 2 * wr : 4 * wr;
+    const uint32_t at2 = kSwiglu ? 2 * RW + 2 * wr : 4 * wr + 2;
+    auto multiply = [&](uint32_t kb, int u) {
+        const uint8_t *la = L.a[u], *lb = L.b[u] + 16 * BT * wc * 128;
+        const i32x8 A[4] = {pf_frag(la + 2048 * at0, off), pf_frag(la + 2048 * at0 + 2048, off),
+                            pf_frag(la + 2048 * at2, off), pf_frag(la + 2048 * at2 + 2048, off)};
+        // PLAIN: a wavefront's rows lie in one 128-row block of scales
+        const float w0 = L.ws[kSwiglu ? 0 : 2 * wr / RW][kb], w1 = kSwiglu ? L.ws[1][kb] : w0;
+#pragma unroll
+        for (int bt = 0; bt < BT; ++bt) {
+            const i32x8 B = pf_frag(lb + 2048 * bt, off);
+            const int sb = L.sb[u][16 * BT * wc + 16 * bt + n];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const f32x4 c = mfma_fp8_sb(A[t], B, f32x4{0.f, 0.f, 0.f, 0.f}, sb);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) tot[t][bt][i] = fmaf(c[i], t < 2 ? w0 : w1, tot[t][bt][i]);
+            }
+        }
+    };
+    // the sets' loads stay in issue order (a wait counts the loads issued after the one it needs)
+    Set P, Q;
+    const uint32_t last = KB - 1;
+    load(P, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    load(Q, min(1u, last));
+    __builtin_amdgcn_sched_barrier(0);
+    stage(P, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    load(P, min(2u, last));
+    __builtin_amdgcn_sched_barrier(0);
+    lds_sync();
+    uint32_t kb = 0;
+    for (; kb + 2 <= KB; kb += 2) {
+        stage(Q, 1);
+        load(Q, min(kb + 3, last));
+        multiply(kb, 0);
+        lds_sync();
+        stage(P, 0);
+        load(P, min(kb + 4, last));
+        multiply(kb + 1, 1);
+        lds_sync();
+    }
+    if (kb < KB) multiply(kb, 0);  // an odd number of k-blocks
+    // epilogue: accumulator lane (g, n) of (A tile t, B tile bt) holds rows 4 g .. 4 g + 3 of A tile
+    // t for activation row 16 bt + n of the wavefront's half
+#pragma unroll
+    for (int bt = 0; bt < BT; ++bt) {
+        const uint32_t r = 16 * BT * wc + 16 * bt + n;
+        if (r >= cnt) continue;
+        if (kSwiglu) {
+            uint16_t *yr = static_cast<uint16_t *>(a.y) + (size_t)(row0 + r) * (a.n / 2) + h0 + 32 * wr + 4 * g;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                uint16_t o[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float gg = tot[t][bt][i], uu = tot[t + 2][bt][i];
+                    o[i] = bf16_rne(gg / (1.0f + expf(-gg)) * uu);
+                }
+                *reinterpret_cast<u32x2 *>(yr + 16 * t) = u32x2{(uint32_t)o[0] | ((uint32_t)o[1] << 16),
+                                                                (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
+            }
+        } else {
+            float *yr = static_cast<float *>(a.y) + (size_t)(row0 + r) * a.n + h0 + 64 * wr + 4 * g;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) *reinterpret_cast<f32x4 *>(yr + 16 * t) = tot[t][bt];
+        }
+    }
+}
+
+// Grid: 8 x ceil(column spans x tiles / 8) workgroups; workgroup b runs on XCD b % 8, and each XCD
+// takes one contiguous range of the (tile, span) list, ordered so that what its workgroups share
+// stays in its L2: by tile, an expert's weights and a tile's activation rows are read into one L2
+// only; by span, a span's weights.
+template <int LAYOUT, bool PAIR>
+__global__ __launch_bounds__(PAIR ? 512 : 256, PAIR ? 2 : 3) void k_pf_qgemm(const PfGemmArgs a) {
+    constexpr int RW = PAIR ? 4 : 2;
+    __shared__ __align__(16) PfLds<64 * RW, PAIR ? 128 : 64> L;
+    const uint32_t nx = a.n / (64 * RW);
+    const uint32_t total = nx * a.ntiles, per = gridDim.x >> 3;
+    const uint32_t id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (id >= total) return;
+    const uint32_t x = a.by_cols ? id / a.ntiles : id % nx, t = a.by_cols ? id % a.ntiles : id / nx;
+    const cu32 *tw = as_const_u32(a.tiles + t);
     const uint64_t w_va = (uint64_t)tw[0] | ((uint64_t)tw[1] << 32);
     const uint64_t s_va = (uint64_t)tw[2] | ((uint64_t)tw[3] << 32);
     const uint32_t row0 = tw[4], cnt = tw[5];
-    const uint32_t KB = a.k / 128;
-    uint32_t ra[2];
-    if (LAYOUT == kPfLayoutSwiglu) {
-        const uint32_t j0 = 64 * blockIdx.x + 16 * w;
-        ra[0] = j0;
-        ra[1] = a.n / 2 + j0;
-    } else {
-        ra[0] = 128 * blockIdx.x + 32 * w;
-        ra[1] = ra[0] + 16;
-    }
-    const uint8_t *wt = reinterpret_cast<const uint8_t *>(w_va);
-    const float *ws = reinterpret_cast<const float *>(s_va);
-    const uint8_t *wa0 = wt + (size_t)(ra[0] + n) * a.k + 16 * g;
-    const uint8_t *wa1 = wt + (size_t)(ra[1] + n) * a.k + 16 * g;
-    const cu32 *ws0 = as_const_u32(ws + (size_t)(ra[0] >> 7) * KB);
-    const cu32 *ws1 = as_const_u32(ws + (size_t)(ra[1] >> 7) * KB);
-    // the activation row this thread stages (rows past cnt are read, never stored)
-    const uint32_t srow_i = row0 + (tid >> 2);
-    const uint32_t src = a.rowidx ? *as_global_u32(a.rowidx + srow_i) : srow_i;
-    const uint8_t *xrow = a.xq + (size_t)src * a.k + 32 * (tid & 3);
-    const uint32_t brow_i = row0 + (tid & 63);
-    const uint32_t bsrc = a.rowidx ? *as_global_u32(a.rowidx + brow_i) : brow_i;
-    const float *xsrow = a.xs + (size_t)bsrc * KB;
-
-    auto load = [&](PfSet &S, uint32_t kb) {
-        S.a[0][0] = __builtin_nontemporal_load(as_global(wa0 + 128 * kb));
-        S.a[0][1] = __builtin_nontemporal_load(as_global(wa0 + 128 * kb + 64));
-        S.a[1][0] = __builtin_nontemporal_load(as_global(wa1 + 128 * kb));
-        S.a[1][1] = __builtin_nontemporal_load(as_global(wa1 + 128 * kb + 64));
-        S.b[0] = *as_global(xrow + 128 * kb);
-        S.b[1] = *as_global(xrow + 128 * kb + 16);
-        S.bs = *as_global_f32(xsrow + kb);
-    };
-    f32x4 tot[2][4];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) tot[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // stage set S (k-block kb, weight scale factor live: 1 or 0) into buffer u, then multiply
-    auto step = [&](const PfSet &S, uint32_t kb, float live, int u) {
-        uint8_t *xbu = xb[u];
-        *reinterpret_cast<u32x4 *>(xbu + (tid >> 2) * kPfRow + 32 * (tid & 3)) = S.b[0];
-        *reinterpret_cast<u32x4 *>(xbu + (tid >> 2) * kPfRow + 32 * (tid & 3) + 16) = S.b[1];
-        if (tid < 64) xsb[u][tid] = S.bs;
-        __syncthreads();
-        const float w0 = __uint_as_float(ws0[kb]) * live, w1 = __uint_as_float(ws1[kb]) * live;
-        const i32x8 A0 = {(int)S.a[0][0].x, (int)S.a[0][0].y, (int)S.a[0][0].z, (int)S.a[0][0].w,
-                          (int)S.a[0][1].x, (int)S.a[0][1].y, (int)S.a[0][1].z, (int)S.a[0][1].w};
-        const i32x8 A1 = {(int)S.a[1][0].x, (int)S.a[1][0].y, (int)S.a[1][0].z, (int)S.a[1][0].w,
-                          (int)S.a[1][1].x, (int)S.a[1][1].y, (int)S.a[1][1].z, (int)S.a[1][1].w};
-#pragma unroll
-        for (int bt = 0; bt < 4; ++bt) {
-            const uint8_t *r = xbu + (16 * bt + n) * kPfRow + 16 * g;
-            const u32x4 b0 = *reinterpret_cast<const u32x4 *>(r);
-            const u32x4 b1 = *reinterpret_cast<const u32x4 *>(r + 64);
-            const i32x8 B = {(int)b0.x, (int)b0.y, (int)b0.z, (int)b0.w, (int)b1.x, (int)b1.y, (int)b1.z, (int)b1.w};
-            const int sb = e8m0_of(xsb[u][16 * bt + n]);
-            const f32x4 c0 = mfma_fp8_sb(A0, B, f32x4{0.f, 0.f, 0.f, 0.f}, sb);
-            const f32x4 c1 = mfma_fp8_sb(A1, B, f32x4{0.f, 0.f, 0.f, 0.f}, sb);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                tot[0][bt][i] = fmaf(c0[i], w0, tot[0][bt][i]);
-                tot[1][bt][i] = fmaf(c1[i], w1, tot[1][bt][i]);
+    if constexpr (PAIR) {
+        // tile j of a run (consecutive tiles of the same weights and contiguous rows): j even takes
+        // tile j + 1 along, j odd is taken by its neighbour
+        const uint32_t lane = lane_id();
+        uint32_t back = 0;
+        for (uint32_t b0 = 1;; b0 += 64) {
+            const uint32_t d = b0 + lane;
+            bool same = d <= t;
+            if (same) {
+                const PfTile *p = a.tiles + (t - d);
+                same = p->w_va == w_va && p->s_va == s_va && p->row0 + 64 * d == row0 && p->cnt == 64;
+            }
+            const uint64_t miss = ~__ballot(same);
+            if (miss) {
+                back += (uint32_t)__builtin_ctzll(miss);
+                break;
+            }
+            back += 64;
+        }
+        if (back & 1) return;
+        if (cnt == 64 && t + 1 < a.ntiles) {
+            const cu32 *nw = as_const_u32(a.tiles + t + 1);
+            if (((uint64_t)nw[0] | ((uint64_t)nw[1] << 32)) == w_va && ((uint64_t)nw[2] | ((uint64_t)nw[3] << 32)) == s_va &&
+                nw[4] == row0 + 64) {
+                pf_qgemm_wg<LAYOUT, RW, 4>(a, L, w_va, s_va, x, row0, 64 + nw[5]);
+                return;
             }
         }
-    };
-    PfSet P, Q;
-    const uint32_t last = KB - 1;
-    load(P, 0);
-    load(Q, min(1u, last));
-    for (uint32_t kb = 0; kb < KB; kb += 2) {
-        step(P, kb, 1.0f, 0);
-        load(P, min(kb + 2, last));
-        step(Q, min(kb + 1, last), kb + 1 < KB ? 1.0f : 0.0f, 1);
-        load(Q, min(kb + 3, last));
     }
-    // epilogue: accumulator lane (g, n) of (A tile i, B tile bt) holds rows 4 g .. 4 g + 3 of A
-    // tile i for activation row 16 bt + n
-#pragma unroll
-    for (int bt = 0; bt < 4; ++bt) {
-        const uint32_t r = 16 * bt + n;
-        if (r >= cnt) continue;
-        if (LAYOUT == kPfLayoutSwiglu) {
-            const uint32_t I = a.n / 2;
-            uint16_t o[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float gg = tot[0][bt][i], uu = tot[1][bt][i];
-                o[i] = bf16_rne(gg / (1.0f + expf(-gg)) * uu);
-            }
-            uint16_t *yr = static_cast<uint16_t *>(a.y) + (size_t)(row0 + r) * I + ra[0] + 4 * g;
-            *reinterpret_cast<u32x2 *>(yr) = u32x2{(uint32_t)o[0] | ((uint32_t)o[1] << 16),
-                                                   (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
-        } else {
-            float *yr = static_cast<float *>(a.y) + (size_t)(row0 + r) * a.n;
-            *reinterpret_cast<f32x4 *>(yr + ra[0] + 4 * g) = tot[0][bt];
-            *reinterpret_cast<f32x4 *>(yr + ra[1] + 4 * g) = tot[1][bt];
-        }
-    }
+    pf_qgemm_wg<LAYOUT, RW, 2>(a, L, w_va, s_va, x, row0, cnt);
 }
 
 // ------------------------------------------------------------------ router logits
@@ -761,11 +848,24 @@ int omega_gpu_pf_qgemm(uint32_t n, uint32_t k, uint32_t layout, uint64_t tiles_v
     a.xq = reinterpret_cast<const uint8_t *>(xq_va);
     a.xs = reinterpret_cast<const float *>(xs_va);
     a.y = reinterpret_cast<void *>(y_va);
+    a.ntiles = ntiles;
+    // fewer activation rows than weight rows of one expert: an XCD that takes column spans reads
+    // less (its spans' weights and the rows) than one that takes tiles (q|k|v at 512 rows 24.2 us
+    // against 25.8; 4096 rows by tile: 106 against 91 us; experts of 2000 tokens by tile 151
+    // against 156 us)
+    a.by_cols = 64ull * ntiles < n;
+    // the paired form halves the weight reads of a run of tiles but leaves one workgroup a CU, so it
+    // takes work for several rounds of 256 (o of 2048 rows, 8192 span-tile-blocks: 50 us against 43;
+    // of 2500 rows 52 either way, of 4096 rows 57 against 73; down of 1250 tokens 81 against 85,
+    // of 3000 tokens 157 against 170). gate|up gains nothing (2000 tokens 172 against 151 us).
+    const bool pair = layout == kPfLayoutPlain && !a.by_cols && n % 256 == 0 &&
+                      (uint64_t)(n / 256) * ntiles * (k / 128) >= 10240;
+    const uint64_t wgs = ((uint64_t)(n / (pair ? 256 : 128)) * ntiles + 7) / 8 * 8;
     return pf_timed(F_SESSION, 1, ns, [&](hipStream_t st) {
-        if (layout == kPfLayoutSwiglu)
-            OMEGA_LAUNCH(k_pf_qgemm<kPfLayoutSwiglu>, dim3(n / 2 / 64, ntiles), dim3(256), 0, st, a);
-        else
-            OMEGA_LAUNCH(k_pf_qgemm<kPfLayoutPlain>, dim3(n / 128, ntiles), dim3(256), 0, st, a);
+        const dim3 grid((uint32_t)wgs), block(pair ? 512 : 256);
+        if (layout == kPfLayoutSwiglu) OMEGA_LAUNCH((k_pf_qgemm<kPfLayoutSwiglu, false>), grid, block, 0, st, a);
+        else if (pair) OMEGA_LAUNCH((k_pf_qgemm<kPfLayoutPlain, true>), grid, block, 0, st, a);
+        else OMEGA_LAUNCH((k_pf_qgemm<kPfLayoutPlain, false>), grid, block, 0, st, a);
         return hipGetLastError();
     });
 }

@@ -177,6 +177,37 @@ def test_qgemm_grouped_swiglu_and_down(omega, oracle, pf):
     DN.free()
 
 
+@pytest.mark.parametrize("n,k,counts", [
+    (128, 128, [1]),                                   # one k-block, one row
+    (384, 384, [64, 1, 63]),                           # odd k-blocks, tiles at and beside 64 rows
+    (256, 256, [17, 0, 65, 128]),
+    # the paired form (256-row workgroups over two tiles of a run): runs of 1 to 5 tiles, full and
+    # partial ends, so pairs start at even and at odd tiles of the table
+    (512, 12288, [64, 128, 65, 1, 192, 320, 129, 63, 256, 200, 64, 300, 130, 640, 511]),
+    (256, 3968, [4096 + 3, 8192]),                     # long runs, an odd number of k-blocks
+])
+def test_qgemm_tile_runs(omega, oracle, pf, n, k, counts):
+    rng = np.random.default_rng(n + k)
+    E, g, bm = len(counts), sum(counts), pf.qgemm_bm()
+    w, s = oracle.synth_fp8(13, 5, E, n, k)
+    T = omega.Fp8Tensor.upload(E, n, k, w, s)
+    q, qs = run_quant(omega, pf, rng.standard_normal((g + bm, k)).astype(np.float32), pf.IN_F32)
+    xq, xs = dev_from(omega, q), dev_from(omega, qs)
+    tiles = pf.build_tiles(bm, [T.entry(e)[0] for e in range(E)], [T.entry(e)[1] for e in range(E)], counts)
+    td = dev_from(omega, tiles.view(np.uint8))
+    yd = dev_from(omega, np.full((g + 1) * n, 7.0, np.float32))
+    pf.qgemm(n, k, pf.PLAIN, td.ptr, len(tiles), 0, xq.ptr, xs.ptr, yd.ptr)
+    y = yd.download(np.float32, (g + 1) * n).reshape(g + 1, n)
+    assert (y[g] == 7.0).all()  # nothing past the last row
+    at = 0
+    for e, c in enumerate(counts):
+        rows = np.unique(np.concatenate([np.arange(min(c, 66)), np.arange(max(0, c - 70), c)])) + at
+        want = dequant_rows(oracle, q[rows], qs[rows]) @ dequant_weights(oracle, w[e:e + 1], s[e:e + 1])[0].T
+        assert c == 0 or rel_err(y[rows], want) <= GEMM_TOL
+        at += c
+    T.free()
+
+
 def sequential_logits(wq_rows, x):
     """logits[r][ex] = the f32 sum from -0.0, in column order, of f32-rounded products, every
     row and expert at once (numpy float32 arithmetic rounds each product and each sum)"""
