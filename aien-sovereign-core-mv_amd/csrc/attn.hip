@@ -673,11 +673,10 @@ __global__ __launch_bounds__(256) void k_paged_items(const PagedItemsArgs a) {
 // ---------------------------------------------------------------- prefill over the fused cache
 // m consecutive tokens at positions pos0 .. pos0 + m - 1 (positions before pos0 already cached):
 // token t's attention is the decode step's at position pos0 + t (per-head q / k RMSNorm, RoPE,
-// its K / V appended, softmax over positions 0 ..= pos0 + t). Three launches: the preparation of
-// every token (q normed and rotated into a scratch row, K and V appended to the cache), the pages
-// of every (token, chunk of kPattnChunk pages, kv head) as one wavefront, and the items combine.
-constexpr uint32_t kPattnChunk = 32;
-
+// its K / V appended, softmax over positions 0 ..= pos0 + t). The K / V append of every token goes
+// first; then one workgroup per (16 query tokens, kv head, chunk of the keys) runs the 128 queries
+// of the kv head's 8 q heads on the bf16 matrix cores. One chunk writes the rows; with more, the
+// partials are merged by k_attn_combine_rows.
 struct PattnArgs {
     const float *qkv = nullptr;  // [m][5120] raw projection rows
     uint8_t *pool = nullptr;
@@ -686,233 +685,297 @@ struct PattnArgs {
     const float *q_norm = nullptr, *k_norm = nullptr;
     const float *rope_cos = nullptr, *rope_sin = nullptr;
     float eps = 1e-6f;
-    float *qn = nullptr;               // [m][32][128] prepared q
-    const uint32_t *items = nullptr;   // [items][4]: first token of the group, chunk, base, chunks
-    float *part = nullptr;             // [items][32][kPartStride]
+    uint32_t nch = 1;            // chunks of the keys per tile
+    float *part = nullptr;       // nch > 1: [m][nch][32][kPartStride]
+    float *out = nullptr;        // nch 1: [m][32][128]
+    float out_scale = 1.0f;
 };
 
-// grid (4 kv heads, m): the kv head's 8 q heads and its K / V row of token t
-__global__ __launch_bounds__(64) void k_pattn_prep(const PattnArgs a) {
-    const uint32_t lane = threadIdx.x, h = blockIdx.x, t = blockIdx.y, pos = a.pos0 + t;
-    const float *row = a.qkv + (size_t)t * 5120;
-    float q0[8], q1[8];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-        q0[r] = *as_global_f32(row + (h * 8 + r) * 128 + lane);
-        q1[r] = *as_global_f32(row + (h * 8 + r) * 128 + 64 + lane);
-    }
-    const float qw0 = *as_global_f32(a.q_norm + lane), qw1 = *as_global_f32(a.q_norm + 64 + lane);
-    const float rc = *as_global_f32(a.rope_cos + (size_t)pos * 64 + lane);
-    const float rs = *as_global_f32(a.rope_sin + (size_t)pos * 64 + lane);
-    float k0 = *as_global_f32(row + 4096 + h * 128 + lane), k1 = *as_global_f32(row + 4096 + h * 128 + 64 + lane);
-    const float v0 = *as_global_f32(row + 4608 + h * 128 + lane);
-    const float v1 = *as_global_f32(row + 4608 + h * 128 + 64 + lane);
+// Workgroup = (page the tokens touch, kv head); wavefront w norms and rotates k of the page's tokens
+// w, w + 4, .. that belong to the call. The V plane is transposed per page, so the tokens' V meet in
+// LDS and a dim's run of tokens goes out in 8-token pieces where the call covers them whole.
+__global__ __launch_bounds__(256) void k_pattn_append(const PattnArgs a) {
+    __shared__ __align__(16) uint16_t vt[128][16];
+    const uint32_t lane = lane_id(), w = threadIdx.x >> 6, h = blockIdx.x & 3, page = (a.pos0 >> 4) + (blockIdx.x >> 2);
+    const uint32_t lo = max(page * 16, a.pos0), hi = min(page * 16 + 16, a.pos0 + a.m);  // positions lo .. hi - 1
     const float kw0 = *as_global_f32(a.k_norm + lane), kw1 = *as_global_f32(a.k_norm + 64 + lane);
-    double ss[8];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) ss[r] = (double)q0[r] * (double)q0[r] + (double)q1[r] * (double)q1[r];
-    const float scale_l = rms_scale(head_sums8(ss, lane), 128, a.eps);
-    float *qo = a.qn + ((size_t)t * 32 + h * 8) * 128;
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-        head_scale_rope(q0[r], q1[r], readlane_f32(scale_l, 8 * r), qw0, qw1, rc, rs, true);
-        qo[r * 128 + lane] = q0[r];
-        qo[r * 128 + 64 + lane] = q1[r];
+    for (uint32_t i = w; i < 16; i += 4) {
+        const uint32_t pos = page * 16 + i;
+        if (pos < lo || pos >= hi) continue;  // uniform per wavefront
+        const float *row = a.qkv + (size_t)(pos - a.pos0) * 5120 + h * 128;
+        float k0 = *as_global_f32(row + 4096 + lane), k1 = *as_global_f32(row + 4096 + 64 + lane);
+        const float v0 = *as_global_f32(row + 4608 + lane), v1 = *as_global_f32(row + 4608 + 64 + lane);
+        const float rc = *as_global_f32(a.rope_cos + (size_t)pos * 64 + lane);
+        const float rs = *as_global_f32(a.rope_sin + (size_t)pos * 64 + lane);
+        const float kscale = rms_scale(wave_sum_f64((double)k0 * (double)k0 + (double)k1 * (double)k1), 128, a.eps);
+        head_scale_rope(k0, k1, kscale, kw0, kw1, rc, rs, true);
+        uint16_t *krow = reinterpret_cast<uint16_t *>(a.pool + kv_row_offset(a.g, page, a.layer, 0, i, h));
+        krow[lane] = bf16_rne(k0);
+        krow[lane + 64] = bf16_rne(k1);
+        vt[lane][i] = bf16_rne(v0);
+        vt[lane + 64][i] = bf16_rne(v1);
     }
-    const float kscale = rms_scale(wave_sum_f64((double)k0 * (double)k0 + (double)k1 * (double)k1), 128, a.eps);
-    head_scale_rope(k0, k1, kscale, kw0, kw1, rc, rs, true);
-    uint16_t *krow = reinterpret_cast<uint16_t *>(a.pool + kv_row_offset(a.g, pos >> 4, a.layer, 0, pos & 15, h));
-    krow[lane] = bf16_rne(k0);
-    krow[lane + 64] = bf16_rne(k1);
-    uint8_t *vplane = a.pool + (uint64_t)(pos >> 4) * a.g.block_stride + (uint64_t)a.layer * a.g.layer_stride +
-                      a.g.plane_stride + (uint64_t)h * kVtHead + (pos & 15) * 2;
-    *reinterpret_cast<uint16_t *>(vplane + lane * 32) = bf16_rne(v0);
-    *reinterpret_cast<uint16_t *>(vplane + (lane + 64) * 32) = bf16_rne(v1);
-}
-
-// one wavefront per (item, kv head): item = (group of TQ consecutive tokens t0 .., chunk c),
-// pages [c C, min(pages, (c + 1) C)) of the group's last token's context; each page is loaded
-// once and serves the group's tokens, token t0 + j masking the positions past its own context
-// pos0 + t0 + j + 1 (a token can see none of a chunk's pages: its state stays empty, m -inf and
-// l 0, and the combine gives it no weight). Item words: t0, c, the group's first partial slot
-// base and its chunk count nch; token j's partial of chunk c is slot base * TQ + j * nch + c, so
-// each token's partials are contiguous for the combine. A tile of TQ > 1 runs its tokens in pairs
-// that share every matrix-core product (pattn_page2: the 16 columns are 2 tokens x 8 heads, so
-// the softmax work per (page, token) halves against TQ = 1, whose 16 columns are one token's 8
-// heads in hi and lo halves), and each page is loaded once for all TQ tokens: TQ 4 for contexts
-// of 1024 and more, 2 from 256, else 1 (a wavefront per token for the parallelism of short
-// prompts).
-constexpr uint32_t kPattnTqLong = 4, kPattnLongCtx = 1024;
-constexpr uint32_t kPattnMidCtx = 256;  // from here one pair of tokens per wavefront
-
-// One page for a pair of query tokens (TQ > 1): the 16 B-columns of S^T = K q^T are the 16
-// queries (token 2 p + n / 8, head n % 8) of the pair, the q operand's hi and lo halves in two
-// product chains into one accumulator, so every lane's four scores are distinct (token, query)
-// entries and the softmax runs once per query; the 16 A-rows of O = P V are the same 16 queries,
-// the probability's hi and lo halves again in two chains. Lane (g, n) holds query n's state (m, l)
-// and rows 4 g + i of O (query 4 g + i, dim 16 nb + n); a query that sees none of the page keeps
-// an empty state (a maximum of -inf is replaced by 0 as the exponent's reference).
-__device__ __forceinline__ void pattn_page2(const DattnPage &T, const bf16x8 (&qh)[4], const bf16x8 (&ql)[4],
-                                            uint32_t tok0, uint32_t ctx_n, uint32_t g, uint32_t n, float &m_l,
-                                            float &l_l, f32x4 (&O)[8]) {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(T.k[ks]), qh[ks], acc, 0, 0, 0);
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(T.k[ks]), ql[ks], acc, 0, 0, 0);
-    float sc[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sc[i] = tok0 + 4 * g + i < ctx_n ? acc[i] * kInvSqrt128 : -INFINITY;
-    const float mx = xor_max<32>(xor_max<16>(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]))));
-    const float m_new = fmaxf(m_l, mx);
-    const float m_ref = m_new == -INFINITY ? 0.f : m_new;
-    float pr[4];
-    float psum = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        pr[i] = expf(sc[i] - m_ref);
-        psum += pr[i];
-    }
-    psum = xor_sum<32>(xor_sum<16>(psum));
-    const float alpha = expf(m_l - m_ref);
-    l_l = l_l * alpha + psum;
-    m_l = m_new;
-    // row 4 g + i is query 4 g + i, whose state lane 4 g + i (lane group 0) holds
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float ai = __shfl(alpha, (int)(4 * g + i));
-#pragma unroll
-        for (int nb = 0; nb < 8; ++nb) O[nb][i] *= ai;
-    }
-    s16x4 ph, pl;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        ph[i] = (short)bf16_split_hi(pr[i]);
-        pl[i] = (short)bf16_split_lo(pr[i]);
-    }
-#pragma unroll
-    for (int nb = 0; nb < 8; ++nb) {
-        O[nb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ph, __builtin_bit_cast(s16x4, T.v[nb]), O[nb], 0, 0, 0);
-        O[nb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pl, __builtin_bit_cast(s16x4, T.v[nb]), O[nb], 0, 0, 0);
-    }
-}
-
-template <uint32_t TQ>
-__global__ __launch_bounds__(64) void k_pattn(const PattnArgs a) {
-    __shared__ __align__(16) uint16_t qhl[TQ][2][8][128];
-    const uint32_t lane = threadIdx.x, h = blockIdx.x & 3, it = blockIdx.x >> 2;
-    const uint32_t g = lane >> 4, n = lane & 15;
-    const uint32_t *iw = a.items + 4 * (size_t)it;
-    const uint32_t t0 = iw[0], c = iw[1], base = iw[2], nch = iw[3];
-    const uint32_t valid = a.m - t0 < TQ ? a.m - t0 : TQ;  // tokens of this group
-    const uint32_t pages = (a.pos0 + t0 + valid + 15) / 16;
-    const uint32_t p_begin = c * kPattnChunk, p_end = min(pages, p_begin + kPattnChunk), last = p_end - 1;
-    uint32_t ctx[TQ];
-#pragma unroll
-    for (uint32_t j = 0; j < TQ; ++j) ctx[j] = j < valid ? a.pos0 + t0 + j + 1 : 0u;
-    DattnArgs d;
-    d.pool = a.pool;
-    d.g = a.g;
-    d.layer = a.layer;
-    DattnPage A, B;
-    if constexpr (TQ == 1) {
-        bf16x8 qop[4];
-        paged_q(a.qn + ((size_t)t0 * 32 + h * 8) * 128, lane, qhl[0], qop);
-        dattn_load(d, h, p_begin, lane, A);
-        dattn_load(d, h, min(p_begin + 1, last), lane, B);
-        float m_l = -INFINITY, l_l = 0.f;
-        f32x4 O[8];
-#pragma unroll
-        for (int nb = 0; nb < 8; ++nb) O[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (uint32_t p = p_begin; p < p_end; p += 2) {
-            const bool has_b = p + 1 < p_end;  // else B is the null page (every score -inf)
-            dattn_page<false, true>(A, qop, p * 16, ctx[0], g, n, m_l, l_l, O);
-            dattn_load(d, h, min(p + 2, last), lane, A);
-            dattn_page<false, true>(B, qop, (p + 1) * 16, has_b ? ctx[0] : 0u, g, n, m_l, l_l, O);
-            dattn_load(d, h, min(p + 3, last), lane, B);
-        }
-        paged_store(a.part + (((size_t)base * TQ + c) * 32 + h * 8) * kPartStride, kPartStride, lane, m_l, l_l, O);
+    __syncthreads();
+    // thread t: dim t / 2, tokens 8 (t % 2) .. +8
+    const uint32_t d = threadIdx.x >> 1, i0 = 8 * (threadIdx.x & 1);
+    uint8_t *vp = a.pool + (uint64_t)page * a.g.block_stride + (uint64_t)a.layer * a.g.layer_stride +
+                  a.g.plane_stride + (uint64_t)h * kVtHead + d * 32 + i0 * 2;
+    if (page * 16 + i0 >= lo && page * 16 + i0 + 8 <= hi) {
+        *reinterpret_cast<u32x4 *>(vp) = *reinterpret_cast<const u32x4 *>(&vt[d][i0]);
     } else {
-        // pairs of tokens share every product (pattn_page2); the 8 q heads of each token are
-        // staged as bf16 hi / lo halves (a missing token repeats the first, never stored)
-        static_assert(TQ % 2 == 0, "query tiles of whole pairs");
-        constexpr uint32_t NP = TQ / 2;
+        for (uint32_t i = i0; i < i0 + 8; ++i)
+            if (page * 16 + i >= lo && page * 16 + i < hi) reinterpret_cast<uint16_t *>(vp)[i - i0] = vt[d][i];
+    }
+}
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+constexpr uint32_t kPattnTile = 16;     // query tokens per workgroup
+constexpr uint32_t kPattnBlock = 32;    // keys per step
+constexpr uint32_t kPattnWgs = 256;     // workgroups that fill the chip (one per CU)
+
+// bf16 pairs hi + lo of two f32 values (to about 2^-17 relative), round to nearest even
+__device__ __forceinline__ void bf16_split_pair(float x, float y, uint32_t &hi, uint32_t &lo) {
+    const bf16x2 h = __builtin_convertvector((f32x2{x, y}), bf16x2);
+    hi = __builtin_bit_cast(uint32_t, h);
+    const bf16x2 l = __builtin_convertvector((f32x2{x - bf16_lo(hi), y - bf16_hi(hi)}), bf16x2);
+    lo = __builtin_bit_cast(uint32_t, l);
+}
+
+// Eight wavefronts: qw = w % 4 owns 32 queries (4 tokens x 8 heads), kw = w / 4 takes every other
+// block of 32 keys; the two halves' states meet in LDS at the end. A block's K and V go through LDS
+// once for the four wavefronts of a half, one block ahead in registers, two LDS buffers, one barrier
+// per step.
+//
+// S^T = K q^T runs as 32x32x16 products with the keys as rows: a lane holds one query's (n = lane %
+// 32) scores of 16 keys, so the softmax needs one exchange with lane ^ 32. Row r of the K operand is
+// key r with bits 2 and 3 swapped; then the lane's accumulators 0..7 and 8..15 are keys 8 hl .. +8 of
+// the block's two pages (hl = lane / 32), which is the B operand of O^T = V^T P^T as it stands: the
+// probabilities never leave their lane, and V^T comes from the transposed plane as 16-byte pieces. q
+// and the probabilities enter as bf16 hi / lo pairs, two product chains into one accumulator.
+//
+// Bounded by the matrix cores and the work per score on the VALU (32 products of 32 cycles and about
+// 150 VALU operations per wavefront and step; the clock drops to 1.9 GHz), not by K / V bytes: 128
+// queries share a block's 16 KiB. At 2500 tokens behind 5000 it runs 0.86 PFLOP/s of bf16 products,
+// where a plain 8192^3 bf16 product reaches 1.2 on this card. Measured (append, attention and
+// combine; wavefronts of up to 4 tokens that read their pages themselves before): 2048 tokens 402
+// -> 98 us, 512 tokens 69 -> 30, 333 tokens behind 3700 202 -> 68, 16 behind 6000 75 -> 35. 64
+// queries a wavefront (4 wavefronts, the q operands in AGPRs) took 149 us at 2048 tokens, four
+// wavefronts a workgroup and two workgroups a CU 108; operands read ahead of their products,
+// wavefront priorities and two score accumulators changed nothing.
+__global__ __launch_bounds__(512, 2) void k_pattn(const PattnArgs a) {
+    __shared__ __align__(16) uint8_t kv[2][2][2][8192];  // [half][buffer][K | V]; also q rows, merge
+    __shared__ float mls[2][4][64];
+    const uint32_t tid = threadIdx.x, lane = lane_id();
+    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), qw = w & 3, kw = w >> 2;
+    const uint32_t n = lane & 31, hl = lane >> 5;
+    const uint32_t tiles = (a.m + kPattnTile - 1) / kPattnTile;
+    const uint32_t h = blockIdx.x & 3, idx = blockIdx.x >> 2;
+    const uint32_t tile = tiles - 1 - idx / a.nch, c = idx % a.nch;  // the longest contexts first
+    const uint32_t t0 = tile * kPattnTile, valid = min(kPattnTile, a.m - t0), ctx = a.pos0 + t0 + valid;
+    const uint32_t blocks = (ctx + kPattnBlock - 1) / kPattnBlock, per = (blocks + a.nch - 1) / a.nch;
+    const uint32_t b0 = min(blocks, c * per), b1 = min(blocks, b0 + per), last_page = (ctx - 1) >> 4;
+
+    // K / V staging: thread t of a half moves K piece t % 16 of token t / 16 and V piece t of both
+    // pages (a page past the context repeats the last one; its keys are masked by position)
+    const uint32_t t = tid & 255;
+    const uint8_t *kbase = a.pool + (uint64_t)a.layer * a.g.layer_stride + (uint64_t)(t >> 4) * a.g.token_stride +
+                           (uint64_t)h * a.g.head_stride + 16 * (t & 15);
+    const uint8_t *vbase = a.pool + (uint64_t)a.layer * a.g.layer_stride + a.g.plane_stride + (uint64_t)h * kVtHead + 16 * t;
+    u32x4 kr[2], vr[2];
+    auto load = [&](uint32_t b) {
 #pragma unroll
-        for (uint32_t j = 0; j < TQ; ++j) {
-            const float *q = a.qn + ((size_t)(j < valid ? t0 + j : t0) * 32 + h * 8) * 128;
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                const float q0 = *as_global_f32(q + r * 128 + lane), q1 = *as_global_f32(q + r * 128 + 64 + lane);
-                qhl[j][0][r][lane] = bf16_split_hi(q0);
-                qhl[j][1][r][lane] = bf16_split_lo(q0);
-                qhl[j][0][r][lane + 64] = bf16_split_hi(q1);
-                qhl[j][1][r][lane + 64] = bf16_split_lo(q1);
-            }
+        for (uint32_t i = 0; i < 2; ++i) {
+            const uint64_t po = (uint64_t)min(2 * b + i, last_page) * a.g.block_stride;
+            kr[i] = *as_global(kbase + po);
+            vr[i] = *as_global(vbase + po);
         }
-        dattn_load(d, h, p_begin, lane, A);
-        dattn_load(d, h, min(p_begin + 1, last), lane, B);
-        __syncthreads();
-        // B operands: column n of pair p is query (token 2 p + n / 8, head n % 8); k-step ks of
-        // lane group g covers dims 32 ks + 8 g .. +8
-        bf16x8 qh[NP][4], ql[NP][4];
-        uint32_t cn[NP];
+    };
+    const uint32_t kslot = (t >> 4) * 256 + (((t & 15) ^ (t >> 4)) << 4);
+    auto stage = [&](int u) {
 #pragma unroll
-        for (uint32_t p = 0; p < NP; ++p) {
-            const uint32_t j = 2 * p + (n >> 3);
-            cn[p] = ctx[0];
-#pragma unroll
-            for (uint32_t jj = 1; jj < TQ; ++jj)
-                if (jj == j) cn[p] = ctx[jj];
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                qh[p][ks] = as_bf16x8(*reinterpret_cast<const u32x4 *>(&qhl[j][0][n & 7][32 * ks + 8 * g]));
-                ql[p][ks] = as_bf16x8(*reinterpret_cast<const u32x4 *>(&qhl[j][1][n & 7][32 * ks + 8 * g]));
-            }
+        for (uint32_t i = 0; i < 2; ++i) {
+            *reinterpret_cast<u32x4 *>(kv[kw][u][0] + 4096 * i + kslot) = kr[i];
+            *reinterpret_cast<u32x4 *>(kv[kw][u][1] + 4096 * i + 16 * t) = vr[i];
         }
-        float m_l[NP], l_l[NP];
-        f32x4 O[NP][8];
+    };
+    load(b0 + kw);
+
+    // the queries: 128 rows (token t0 + r / 8, head r % 8) through LDS, piece p at slot p ^ (r % 32)
+    uint8_t *qs = &kv[0][0][0][0];
 #pragma unroll
-        for (uint32_t p = 0; p < NP; ++p) {
-            m_l[p] = -INFINITY;
-            l_l[p] = 0.f;
+    for (uint32_t i = 0; i < 8; ++i) {
+        const uint32_t p = tid + 512 * i, r = p >> 5, pc = p & 31, tok = t0 + min(r >> 3, valid - 1);
+        *reinterpret_cast<u32x4 *>(qs + r * 512 + ((pc ^ (r & 31)) << 4)) =
+            *as_global(a.qkv + (size_t)tok * 5120 + (h * 8 + (r & 7)) * 128 + 4 * pc);
+    }
+    lds_sync();
+    const uint32_t j = 4 * qw + (n >> 3), head = n & 7;          // the lane's query: token t0 + j
+    const uint32_t pos = a.pos0 + t0 + min(j, valid - 1);
+    bf16x8 qh[8], ql[8];                                         // dims 16 ks + 8 hl .. +8
+    {
+        float v[8][8];
 #pragma unroll
-            for (int nb = 0; nb < 8; ++nb) O[p][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-        for (uint32_t pg = p_begin; pg < p_end; pg += 2) {
-            const bool has_b = pg + 1 < p_end;  // else B is the null page (every score -inf)
+        for (uint32_t ks = 0; ks < 8; ++ks)
 #pragma unroll
-            for (uint32_t p = 0; p < NP; ++p) pattn_page2(A, qh[p], ql[p], pg * 16, cn[p], g, n, m_l[p], l_l[p], O[p]);
-            dattn_load(d, h, min(pg + 2, last), lane, A);
+            for (uint32_t q = 0; q < 2; ++q) {
+                const f32x4 x = *reinterpret_cast<const f32x4 *>(qs + (32 * qw + n) * 512 + (((4 * ks + 2 * hl + q) ^ n) << 4));
 #pragma unroll
-            for (uint32_t p = 0; p < NP; ++p)
-                pattn_page2(B, qh[p], ql[p], (pg + 1) * 16, has_b ? cn[p] : 0u, g, n, m_l[p], l_l[p], O[p]);
-            dattn_load(d, h, min(pg + 3, last), lane, B);
-        }
-        // partials: row 4 g + i of pair p is query 4 g + i (token 2 p + g / 2, head 4 (g % 2) + i);
-        // lanes 0..15 hold query n's (m, l). Token j's partial of chunk c is slot base * TQ + j *
-        // nch + c, its head r at r * kPartStride (m, l, -, -, o[128]).
-#pragma unroll
-        for (uint32_t p = 0; p < NP; ++p) {
-            const uint32_t jo = 2 * p + (g >> 1);
-            if (jo < valid) {
-                float *pt = a.part + (((size_t)base * TQ + jo * nch + c) * 32 + h * 8) * kPartStride;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float *pp = pt + (size_t)(4 * (g & 1) + i) * kPartStride + 4;
-#pragma unroll
-                    for (int nb = 0; nb < 8; ++nb) pp[16 * nb + n] = O[p][nb][i];
-                }
+                for (int e = 0; e < 4; ++e) v[ks][4 * q + e] = x[e];
             }
-            const uint32_t jm = 2 * p + (n >> 3);
-            if (lane < 16 && jm < valid) {
-                float *pp = a.part + (((size_t)base * TQ + jm * nch + c) * 32 + h * 8 + (n & 7)) * kPartStride;
-                pp[0] = m_l[p];
-                pp[1] = l_l[p];
+        double ss = 0.0;
+#pragma unroll
+        for (uint32_t ks = 0; ks < 8; ++ks)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += (double)v[ks][e] * (double)v[ks][e];
+        const float scale = rms_scale(pair_sum<32>(ss, ss), 128, a.eps);
+#pragma unroll
+        for (uint32_t ks = 0; ks < 4; ++ks)
+#pragma unroll
+            for (uint32_t q = 0; q < 2; ++q) {
+                const uint32_t d = 16 * ks + 8 * hl + 4 * q;
+                const f32x4 w0 = *as_global_f32x4(a.q_norm + d), w1 = *as_global_f32x4(a.q_norm + 64 + d);
+                const f32x4 rc = *as_global_f32x4(a.rope_cos + (size_t)pos * 64 + d);
+                const f32x4 rs = *as_global_f32x4(a.rope_sin + (size_t)pos * 64 + d);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    head_scale_rope(v[ks][4 * q + e], v[ks + 4][4 * q + e], scale, w0[e], w1[e], rc[e], rs[e], true);
             }
+#pragma unroll
+        for (uint32_t ks = 0; ks < 8; ++ks) {
+            u32x4 hi, lo;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                uint32_t x, y;
+                bf16_split_pair(v[ks][2 * e], v[ks][2 * e + 1], x, y);
+                hi[e] = x;
+                lo[e] = y;
+            }
+            qh[ks] = as_bf16x8(hi);
+            ql[ks] = as_bf16x8(lo);
         }
     }
+    lds_sync();  // the q rows are read
+
+    constexpr float kC = kInvSqrt128 * 1.4426950408889634f;      // exp(s / sqrt 128) = 2^(kC s)
+    float m_l = -INFINITY, l_l = 0.f;                            // l: this lane's keys only
+    f32x16 O[4];                                                 // O[dt][i]: dim 32 dt + 8 (i / 4) + 4 hl + i % 4
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) O[dt][i] = 0.f;
+    const uint32_t kt = (n & 0x13) | ((n & 4) << 1) | ((n & 8) >> 1);  // the key of K row n
+    const uint32_t koff = kt * 256, kx = kt & 15;
+    auto compute = [&](int u, uint32_t b) {
+        const uint8_t *kb = kv[kw][u][0] + koff, *vb = kv[kw][u][1] + n * 32 + 16 * hl;
+        f32x16 s;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = 0.f;
+#pragma unroll
+        for (uint32_t ks = 0; ks < 8; ++ks) {
+            const bf16x8 k = as_bf16x8(*reinterpret_cast<const u32x4 *>(kb + (((2 * ks + hl) ^ kx) << 4)));
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k, qh[ks], s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k, ql[ks], s, 0, 0, 0);
+        }
+        if (kPattnBlock * b + kPattnBlock > a.pos0 + t0 + 1) {   // some query does not see some key
+            asm volatile("");                                    // stays a branch: most blocks skip it
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                if (kPattnBlock * b + 16 * (i >> 3) + 8 * hl + (i & 7) > pos) s[i] = -INFINITY;
+        }
+        float mx = s[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+        mx = xor_max<32>(mx);
+        const float m_new = fmaxf(m_l, mx);
+        const float m_ref = m_new == -INFINITY ? 0.f : m_new;
+        const float mc = -m_ref * kC;
+        if (__any(m_new != m_l)) {                               // else every factor is 1
+            const float alpha = __builtin_amdgcn_exp2f(fmaf(m_l, kC, mc));
+            l_l *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) O[dt][i] *= alpha;
+            m_l = m_new;
+        }
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            u32x4 hi, lo;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float p0 = __builtin_amdgcn_exp2f(fmaf(s[8 * kk + 2 * e], kC, mc));
+                const float p1 = __builtin_amdgcn_exp2f(fmaf(s[8 * kk + 2 * e + 1], kC, mc));
+                l_l += p0 + p1;
+                uint32_t x, y;
+                bf16_split_pair(p0, p1, x, y);
+                hi[e] = x;
+                lo[e] = y;
+            }
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) {
+                const bf16x8 v = as_bf16x8(*reinterpret_cast<const u32x4 *>(vb + 4096 * kk + 1024 * dt));
+                O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, as_bf16x8(hi), O[dt], 0, 0, 0);
+                O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, as_bf16x8(lo), O[dt], 0, 0, 0);
+            }
+        }
+    };
+    const uint32_t steps = (b1 - b0 + 1) / 2;
+    stage(0);
+    load(b0 + kw + 2);
+    lds_sync();
+    for (uint32_t i = 0; i < steps; ++i) {
+        const uint32_t b = b0 + kw + 2 * i;
+        const int u = i & 1;
+        stage(u ^ 1);
+        load(b + 4);
+        if (b < b1) compute(u, b);  // uniform per wavefront
+        lds_sync();
+    }
+    // the two halves' states, lane by lane
+    float *mo = reinterpret_cast<float *>(&kv[0][0][0][0]) + qw * 4096 + lane;
+    if (kw == 1) {
+        mls[0][qw][lane] = m_l;
+        mls[1][qw][lane] = l_l;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) mo[64 * (16 * dt + i)] = O[dt][i];
+    }
+    lds_sync();
+    if (kw == 1) return;
+    {
+        const float m1 = mls[0][qw][lane], M = fmaxf(m_l, m1), mc = M == -INFINITY ? 0.f : -M * kC;
+        const float w0 = __builtin_amdgcn_exp2f(fmaf(m_l, kC, mc)), w1 = __builtin_amdgcn_exp2f(fmaf(m1, kC, mc));
+        m_l = M;
+        l_l = fmaf(l_l, w0, mls[1][qw][lane] * w1);
+        l_l = xor_sum<32>(l_l);
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) O[dt][i] = fmaf(O[dt][i], w0, mo[64 * (16 * dt + i)] * w1);
+    }
+    if (j >= valid) return;
+    float *dst;
+    float f = 1.f;
+    if (a.nch == 1) {
+        dst = a.out + (size_t)(t0 + j) * 4096 + (h * 8 + head) * 128;
+        f = a.out_scale / l_l;
+    } else {
+        float *pp = a.part + (((size_t)(t0 + j) * a.nch + c) * 32 + h * 8 + head) * kPartStride;
+        if (hl == 0) {
+            pp[0] = m_l * kInvSqrt128;
+            pp[1] = l_l;
+        }
+        dst = pp + 4;
+    }
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<f32x4 *>(dst + 32 * dt + 8 * q + 4 * hl) =
+                f32x4{O[dt][4 * q] * f, O[dt][4 * q + 1] * f, O[dt][4 * q + 2] * f, O[dt][4 * q + 3] * f};
 }
 
 // ---------------------------------------------------------------- KV park / restore (extension)
@@ -1368,15 +1431,15 @@ hipError_t launch_attn_combine(const CombineArgs &a, hipStream_t st) {
 // the items' (m, l) are read by thread j % 256 of item j, their weights exp(m - M) staged in LDS;
 // thread t then sums dims 4 (t % 32) .. +3 over the items j = t / 32 (mod 8) and the 8 groups
 // meet in LDS in a fixed order; 16 lanes split the head's row.
-// The f32 rows of sequences (prefill tokens) that have at most 64 partials each: one wavefront per
-// (sequence, q head), lane j holding partial j's (m, l), lane l dims l and l + 64; the partials
+// The f32 rows of sequences (prefill tokens) of nch <= 64 partials each: one wavefront per (sequence,
+// q head), lane j holding partial j's (m, l), lane l dims l and l + 64; the partials
 // merge in item order (out = sum w_j o_j / sum w_j l_j with w_j = exp(m_j - max m), times
 // out_scale). A token always has a partial that sees its own position, so the maximum is finite.
-__global__ __launch_bounds__(256) void k_attn_combine_rows(const CombineItemsArgs a, uint32_t seqs) {
+__global__ __launch_bounds__(256) void k_attn_combine_rows(const CombineItemsArgs a, uint32_t seqs, uint32_t nch) {
     const uint32_t lane = lane_id(), wv = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (wv >= seqs * 32) return;  // uniform per wavefront
     const uint32_t s = wv >> 5, head = wv & 31;
-    const uint32_t off = a.item_off[s], n = a.item_off[s + 1] - off;  // 1 ..= 64
+    const uint32_t off = s * nch, n = nch;  // 1 ..= 64
     constexpr size_t kItem = 32 * (size_t)kPartStride;                // floats from one item to the next
     const float *base = a.part + ((size_t)off * 32 + head) * kPartStride;
     const u32x2 ml = *as_global_u32x2(base + min(lane, n - 1) * kItem);
@@ -1944,42 +2007,40 @@ int omega_gpu_decode_attn_cache_import_dev(OmegaGpuDecodeAttnCache *c, uint32_t 
                     kvio_none, kvio_none);
 }
 
-// Sub-batches of at most kPattnSub tokens bound the prefill attention's scratch.
-constexpr uint32_t kPattnSub = 1024;
+// Sub-batches of at most kPattnSub tokens (a multiple of the query tile): a launch's K / V append
+// goes before its attention, and a sub-batch sees the ones before it in the cache.
+constexpr uint32_t kPattnSub = 4096;
 
-// Scratch layout of one prefill attention call of m tokens from pos0: the prepared q rows of a
-// sub-batch, its item plan and token offsets, and the partials of its items. Sized from the
-// call's own last position, so a short prompt on a large cache asks for little.
-struct PattnScratch {
-    size_t qn, items, off, part;
-    size_t total() const { return qn + items + off + part; }
-};
-static PattnScratch pattn_scratch(uint32_t pos0, uint32_t m) {
-    const uint32_t sub = std::min(kPattnSub, m);
-    const uint32_t max_chunks = ((pos0 + m + 15) / 16 + kPattnChunk - 1) / kPattnChunk;
-    const size_t max_items = (size_t)sub * max_chunks;
-    PattnScratch s;
-    s.qn = (size_t)sub * 32 * 128 * 4;
-    s.items = (max_items * 16 + 255) / 256 * 256;
-    s.off = ((sub + 1) * 4 + 255) / 256 * 256;
-    s.part = (max_items * 32 * kPartStride * 4 + 255) / 256 * 256;
-    return s;
+// Chunks of the keys for a call of m tokens from pos0: with fewer workgroups than CUs the keys are
+// cut, into pieces of at least 512 keys (16 blocks), until the workgroups fill the chip. A tile
+// that fills it whole writes its rows directly (2048 tokens: no partials to write and read back).
+static uint32_t pattn_chunks(uint32_t pos0, uint32_t m) {
+    const uint32_t wgs = 4 * ((m + kPattnTile - 1) / kPattnTile);
+    if (2 * wgs > kPattnWgs) return 1;
+    const uint32_t by_len = ((pos0 + m + 15) / 16 + 31) / 32;
+    return std::max(1u, std::min({kPattnWgs / wgs, by_len, 64u}));
+}
+
+// The scratch that a prefill attention call of m tokens from pos0 asks for. The serving reservation
+// and its seal are written against this size (a sealed library refuses a call that asks for more
+// than it holds), so it stays what it was when a call held 1024 prepared query rows, their plan and
+// a partial per token and 512 keys. The partials of this form (at most 512 tokens in at most that
+// many chunks) fit in it.
+static size_t pattn_scratch(uint32_t pos0, uint32_t m) {
+    const size_t sub = std::min(1024u, m), chunks = ((pos0 + m + 15) / 16 + 31) / 32, items = sub * chunks;
+    auto up = [](size_t v) { return (v + 255) / 256 * 256; };
+    return sub * 32 * 128 * 4 + up(items * 16) + up((sub + 1) * 4) + up(items * 32 * kPartStride * 4);
 }
 
 // The prefill attention of m tokens on the fused cache (both entries): qkv_dev [m][5120] and
-// out_dev [m][4096] device rows. Sub-batches of at most kPattnSub tokens; each runs the
-// preparation (K / V of its tokens appended), the page items and their combine. The working set
-// is the first pattn_scratch(pos0, m).total() bytes of the context's scratch.
+// out_dev [m][4096] device rows. The partials sit at the start of the context's scratch, within
+// its first pattn_scratch(pos0, m) bytes.
 static int prefill_attn_run(OmegaGpuDecodeAttnCache *c, uint32_t layer, uint32_t pos0, uint32_t m,
                             const float *qkv_dev, float eps, float out_scale, float *out_dev,
                             OmegaGpuPrefillAttnInfo *info, const uint64_t t_call) {
     Ctx *cx = ctx(F_DATTN);
     if (!cx) return OMEGA_GPU_CHIP_FAIL;
-    constexpr uint32_t kSub = kPattnSub;
-    const PattnScratch sz = pattn_scratch(pos0, m);
-    if (!ensure_scratch(F_DATTN, cx, sz.total())) return OMEGA_GPU_CHIP_FAIL;
-    const size_t qn_bytes = sz.qn, item_bytes = sz.items, off_bytes = sz.off;
-    uint8_t *base = static_cast<uint8_t *>(cx->scratch);
+    if (!ensure_scratch(F_DATTN, cx, pattn_scratch(pos0, m))) return OMEGA_GPU_CHIP_FAIL;
     PattnArgs a;
     a.pool = c->pool;
     a.g = c->g;
@@ -1989,67 +2050,33 @@ static int prefill_attn_run(OmegaGpuDecodeAttnCache *c, uint32_t layer, uint32_t
     a.rope_cos = c->rope_cos;
     a.rope_sin = c->rope_sin;
     a.eps = eps;
-    a.qn = reinterpret_cast<float *>(base);
-    uint32_t *ditems = reinterpret_cast<uint32_t *>(base + qn_bytes);
-    uint32_t *doff = reinterpret_cast<uint32_t *>(base + qn_bytes + item_bytes);
-    a.items = ditems;
-    a.part = reinterpret_cast<float *>(base + qn_bytes + item_bytes + off_bytes);
-    std::vector<uint32_t> items, off;
+    a.part = static_cast<float *>(cx->scratch);
+    a.out_scale = out_scale;
     uint32_t total_items = 0, widest = 0;
     OMEGA_HIP(F_DATTN, hipEventRecord(cx->ev0, cx->stream));
-    for (uint32_t t0 = 0; t0 < m; t0 += kSub) {
-        const uint32_t mm = std::min(kSub, m - t0);
-        items.clear();
-        off.assign(mm + 1, 0);
-        // groups of tq tokens share their page loads; each group's chunks follow its last token's
-        // context, and token j of a group owns the partial slots base * tq + j * nch + chunk (kSub
-        // is a multiple of tq, so a group never spans sub-batches)
-        const uint32_t ctx_end = pos0 + t0 + mm;
-        const uint32_t tq = ctx_end >= kPattnLongCtx ? kPattnTqLong : ctx_end >= kPattnMidCtx ? 2u : 1u;
-        uint32_t base = 0;
-        for (uint32_t g0 = 0; g0 < mm; g0 += tq) {
-            const uint32_t valid = std::min(tq, mm - g0);
-            const uint32_t pages = (pos0 + t0 + g0 + valid + 15) / 16, nch = (pages + kPattnChunk - 1) / kPattnChunk;
-            for (uint32_t j = 0; j < valid; ++j) off[g0 + j] = base * tq + j * nch;
-            off[mm] = base * tq + valid * nch;
-            for (uint32_t ch = 0; ch < nch; ++ch) {
-                items.push_back(g0);
-                items.push_back(ch);
-                items.push_back(base);
-                items.push_back(nch);
-            }
-            base += nch;
-            widest = std::max(widest, nch);
-        }
-        const uint32_t n = (uint32_t)(items.size() / 4);
-        total_items += n;
-        OMEGA_HIP(F_DATTN, hipMemcpyAsync(ditems, items.data(), items.size() * 4, hipMemcpyHostToDevice, cx->stream));
-        OMEGA_HIP(F_DATTN, hipMemcpyAsync(doff, off.data(), off.size() * 4, hipMemcpyHostToDevice, cx->stream));
+    for (uint32_t t0 = 0; t0 < m; t0 += kPattnSub) {
+        const uint32_t mm = std::min(kPattnSub, m - t0);
         a.qkv = qkv_dev + (size_t)t0 * 5120;
+        a.out = out_dev + (size_t)t0 * 4096;
         a.pos0 = pos0 + t0;
         a.m = mm;
-        OMEGA_LAUNCH(k_pattn_prep, dim3(4, mm), dim3(64), 0, cx->stream, a);
+        a.nch = pattn_chunks(a.pos0, mm);
+        const uint32_t pages = ((a.pos0 + mm - 1) >> 4) - (a.pos0 >> 4) + 1;
+        const uint32_t items = (mm + kPattnTile - 1) / kPattnTile * a.nch;
+        total_items += items;
+        widest = std::max(widest, a.nch);
+        OMEGA_LAUNCH(k_pattn_append, dim3(4 * pages), dim3(256), 0, cx->stream, a);
         OMEGA_HIP(F_DATTN, hipGetLastError());
-        if (tq == 1)
-            OMEGA_LAUNCH(k_pattn<1>, dim3(4 * n), dim3(64), 0, cx->stream, a);
-        else if (tq == 2)
-            OMEGA_LAUNCH(k_pattn<2>, dim3(4 * n), dim3(64), 0, cx->stream, a);
-        else
-            OMEGA_LAUNCH(k_pattn<kPattnTqLong>, dim3(4 * n), dim3(64), 0, cx->stream, a);
+        OMEGA_LAUNCH(k_pattn, dim3(4 * items), dim3(512), 0, cx->stream, a);
         OMEGA_HIP(F_DATTN, hipGetLastError());
-        CombineItemsArgs cb;
-        cb.part = a.part;
-        cb.item_off = doff;
-        cb.out = out_dev + (size_t)t0 * 4096;
-        cb.out_scale = out_scale;
-        if (widest <= 64) {  // a wavefront per (token, q head)
-            OMEGA_LAUNCH(k_attn_combine_rows, dim3((mm * 32 + 3) / 4), dim3(256), 0, cx->stream, cb, mm);
+        if (a.nch > 1) {  // a wavefront per (token, q head)
+            CombineItemsArgs cb;
+            cb.part = a.part;
+            cb.out = a.out;
+            cb.out_scale = out_scale;
+            OMEGA_LAUNCH(k_attn_combine_rows, dim3((mm * 32 + 3) / 4), dim3(256), 0, cx->stream, cb, mm, a.nch);
             OMEGA_HIP(F_DATTN, hipGetLastError());
-        } else {
-            OMEGA_HIP(F_DATTN, launch_attn_combine_items(cb, mm, cx->stream));
         }
-        // the host plan is read by the copies above before the next sub-batch rewrites it
-        OMEGA_HIP(F_DATTN, hipStreamSynchronize(cx->stream));
     }
     OMEGA_HIP(F_DATTN, hipEventRecord(cx->ev1, cx->stream));
     OMEGA_HIP(F_DATTN, hipEventSynchronize(cx->ev1));
@@ -2063,9 +2090,9 @@ static int prefill_attn_run(OmegaGpuDecodeAttnCache *c, uint32_t layer, uint32_t
         info->chunks = total_items;
         info->grid_x = 4 * total_items;
         info->grid_y = 1;
-        info->threads = 64;
+        info->threads = 512;
         info->splits = widest;
-        info->per_split = kPattnChunk * 16;
+        info->per_split = ((pos0 + m + kPattnBlock - 1) / kPattnBlock + widest - 1) / widest * kPattnBlock;
         info->elapsed_ns = (uint64_t)((double)ms * 1e6);
         info->call_ns = now_ns() - t_call;
         info->kernel_cache_hit = 1;
@@ -2102,7 +2129,7 @@ int omega_gpu_prefill_attn(OmegaGpuDecodeAttnCache *c, uint32_t layer, uint32_t 
     // the q|k|v and out rows sit in the context's scratch after the run's own working set, so the
     // serving seal and the allocation counters cover this entry like every other host entry
     const size_t qb = (size_t)m * 5120 * 4, ob = (size_t)m * 4096 * 4;
-    const size_t run_bytes = (pattn_scratch(pos0, m).total() + 255) / 256 * 256;
+    const size_t run_bytes = (pattn_scratch(pos0, m) + 255) / 256 * 256;
     if (!ensure_scratch(F_DATTN, cx, run_bytes + qb + ob)) return OMEGA_GPU_CHIP_FAIL;
     if (!ensure_pinned(F_DATTN, cx, std::max(qb, ob))) return OMEGA_GPU_CHIP_FAIL;
     void *d = static_cast<uint8_t *>(cx->scratch) + run_bytes;

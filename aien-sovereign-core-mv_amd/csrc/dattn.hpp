@@ -46,9 +46,7 @@ __device__ __forceinline__ void dattn_load(const DattnArgs &a, uint32_t h, uint3
 // One online-softmax step over a page whose first token is tok0 (< pos). The online state of
 // head n % 8 (m, l) sits in every lane of column n; O[nb][i] is row 4 g + i (head (4 g + i) % 8,
 // hi half for g < 2, lo half otherwise), dim 16 nb + n.
-// GUARD: the page may hold no valid token for a running state that has seen none either (the
-// prefill's query tiles), so a maximum of -inf is replaced by 0 as the exponent's reference.
-template <bool FIRST, bool GUARD = false>  // FIRST: no earlier page (the running state starts here)
+template <bool FIRST>  // FIRST: no earlier page (the running state starts here)
 __device__ __forceinline__ void dattn_page(const DattnPage &T, const bf16x8 (&qop)[4], uint32_t tok0,
                                            uint32_t pos, uint32_t g, uint32_t n, float &m_l, float &l_l,
                                            f32x4 (&O)[8]) {
@@ -64,20 +62,19 @@ __device__ __forceinline__ void dattn_page(const DattnPage &T, const bf16x8 (&qo
     }
     // max and sum over the four lane groups (rows) of a column: row swaps, no LDS
     const float mx = xor_max<32>(xor_max<16>(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]))));
-    const float m_new = FIRST ? mx : fmaxf(m_l, mx);  // finite unless GUARD: token tok0 is valid
-    const float m_ref = GUARD && m_new == -INFINITY ? 0.f : m_new;
+    const float m_new = FIRST ? mx : fmaxf(m_l, mx);  // finite: token tok0 is valid
     float pr[4];
     float psum = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        pr[i] = expf(sc[i] - m_ref);
+        pr[i] = expf(sc[i] - m_new);
         psum += pr[i];
     }
     psum = xor_sum<32>(xor_sum<16>(psum));
     if (FIRST) {
         l_l = psum;
     } else {
-        const float alpha = expf(m_l - m_ref);
+        const float alpha = expf(m_l - m_new);
         l_l = l_l * alpha + psum;
         // accumulator row 4 g + i belongs to head (4 g + i) % 8: head i for even g, 4 + i for
         // odd g, whose alpha every row's lane (head) holds

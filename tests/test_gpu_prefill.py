@@ -309,6 +309,44 @@ def test_prefill_attention_equals_the_decode_attention(omega, oracle, pf, N, fir
     b.free()
 
 
+@pytest.mark.parametrize("pos0,m", [
+    (0, 1), (0, 15), (0, 17), (0, 33),        # less than, at and past a tile of 16 tokens / 32 keys
+    (5, 16), (31, 40),                        # first and last pages shared with earlier positions
+    (500, 65), (2040, 130), (3000, 3),        # the keys cut in chunks, some past a short tile's end
+])
+def test_prefill_attention_tile_edges(omega, oracle, pf, pos0, m):
+    rng = np.random.default_rng(1000 + pos0 + m)
+    eps, maxp = 1e-6, omega.round_max_pos(pos0 + m + 17)
+    qn, kn = (1 + 0.1 * rng.standard_normal((2, 128))).astype(np.float32)
+    c, d = omega.DecodeAttnCache(1, maxp, 1e6), oracle.Dattn(1, maxp, 1e6)
+    c.set_norms(0, qn, kn)
+    d.set_norms(0, qn, kn)
+    past = -(-(pos0 + m) // 16) * 16          # NaN in the pages that no query sees
+    nan = np.full((maxp - past, 128), 0x7fc0, np.uint16)
+    for h in range(4):
+        c.write_rows(0, h, past, nan, nan)
+        if pos0:
+            k, v = (oracle.f32_to_bf16(rng.standard_normal((pos0, 128)).astype(np.float32)) for _ in range(2))
+            c.write_rows(0, h, 0, k, v)
+            d.write_rows(0, h, 0, k, v)
+    qkv = rng.standard_normal((m, 5120)).astype(np.float32)
+    out, _ = pf.PrefillAttention(c).attend(0, pos0, m, qkv, eps, 0.5)
+    for t in range(m):
+        want = 0.5 * d.attend(0, pos0 + t, qkv[t], eps)
+        # q and the probabilities as bf16 pairs (2^-17 each): scores of up to about 12 move by 1e-4,
+        # and a K value on a bf16 rounding boundary by 2^-9 of itself
+        assert rel_err(out[t], want) <= 5e-4, t
+    for h in range(4):
+        for p in {pos0, pos0 + m // 2, pos0 + m - 1}:
+            for x, y in zip(c.read_row(0, h, p), d.read_row(0, h, p)):
+                np.testing.assert_array_equal(x, y)
+        if pos0:
+            for x, y in zip(c.read_row(0, h, pos0 - 1), d.read_row(0, h, pos0 - 1)):
+                np.testing.assert_array_equal(x, y)  # the positions before the call stay
+        assert (c.read_row(0, h, past)[0] == 0x7fc0).all()
+    c.free()
+
+
 def test_prefill_attention_refusals(omega, pf):
     c = omega.DecodeAttnCache(1, 256, 1e6)
     att = pf.PrefillAttention(c)
