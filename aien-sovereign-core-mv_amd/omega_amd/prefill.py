@@ -312,16 +312,25 @@ class WholePromptPrefill:
         kmax = max(h, qd)
         mt = -(-m // self.t) * self.t
         max_tiles = -(-g // bm) + e
+        # the layer's plan, written by the host next to the logits it is made from and moved by one
+        # copy (byte offsets): activation row of each grouped row, grouped row and weight of each
+        # (token, slot), the tile tables of gate|up and down
+        up16 = lambda v: (v + 15) // 16 * 16
+        at = [0]
+        for nb in ((g + bm) * 4, g * 4, g * 4, max_tiles * TILE_BYTES, max_tiles * TILE_BYTES):
+            at.append(at[-1] + up16(nb))
+        base = up16(mt * e * 4)
+        dense_tiles = len(self.layers) * 2 * -(-m // bm)
         # HOST buffers are the CPU's side (written or read in place); the kernels read and write
         # DEVICE buffers, and the copies between them are DMA (omega_gpu_pf_copy_va)
-        b = dict(m=m, max_tiles=max_tiles,
-                 stage=PfMem(max(mt * max(h, e), m * qkv_n, g * h) * 4 + g * 8, host=True),
+        b = dict(m=m, max_tiles=max_tiles, plan_at=at, plan_stage=base,
+                 stage=PfMem(max(max(mt * max(h, e), m * qkv_n, g * h) * 4 + g * 8, base + at[-1],
+                                 dense_tiles * TILE_BYTES), host=True),
                  x=PfMem(m * h * 4), xin=PfMem(mt * h * 4), xq=PfMem((m + bm) * kmax), xs=PfMem((m + bm) * (kmax // BLOCK) * 4),
                  qkv=PfMem(m * qkv_n * 4), att=PfMem(m * qd * 4), oproj=PfMem(m * h * 4),
-                 logits=PfMem(mt * e * 4), rowidx=PfMem((g + bm) * 4),
-                 act=PfMem(g * i * 2), aq=PfMem((g + bm) * i), a_s=PfMem((g + bm) * (i // BLOCK) * 4),
-                 down=PfMem(g * h * 4), inv=PfMem(g * 4), wts=PfMem(g * 4), moe=PfMem(m * h * 4),
-                 tiles=PfMem(3 * max_tiles * TILE_BYTES, host=True))
+                 logits=PfMem(mt * e * 4), act=PfMem(g * i * 2), aq=PfMem((g + bm) * i),
+                 a_s=PfMem((g + bm) * (i // BLOCK) * 4), down=PfMem(g * h * 4), moe=PfMem(m * h * 4),
+                 plan=PfMem(at[-1]), dense=PfMem(dense_tiles * TILE_BYTES))
         self.bufs = b
         return b
 
@@ -335,24 +344,48 @@ class WholePromptPrefill:
         st[:arr.nbytes] = arr.view(np.uint8).reshape(-1)
         copy_va(dst.va, self.bufs["stage"].va, nb)
 
-    def _down(self, src, dtype, count):
-        nb = (count * np.dtype(dtype).itemsize + 15) // 16 * 16
-        if nb > self.bufs["stage"].nbytes or nb > src.nbytes:
+    def _down(self, src, dtype, count, first=0):
+        """values first .. first + count - 1 of a device buffer, as a view of the staging buffer (the
+        next staging copy overwrites it)"""
+        size = np.dtype(dtype).itemsize
+        nb = (count * size + 15) // 16 * 16
+        if nb > self.bufs["stage"].nbytes or first * size + nb > src.nbytes:
             raise OmegaGpuError(-1, f"staging copy of {nb} bytes exceeds its buffers")
-        copy_va(self.bufs["stage"].va, src.va, nb)
-        return self.bufs["stage"].host(dtype)[:count].copy()
+        copy_va(self.bufs["stage"].va, src.va + first * size, nb)
+        return self.bufs["stage"].host(dtype)[:count]
 
-    def _put_tiles(self, b, region, ws, counts):
-        """the tile table of (weights, scales) addresses `ws` over `counts` rows per expert, built
-        by the library's builder straight into the pinned table region"""
-        w, sc = ws
-        c = np.ascontiguousarray(counts, np.uint32)
-        off = region * b["max_tiles"] * TILE_BYTES
-        n = lib().omega_gpu_pf_qgemm_tiles_va(len(c), w.ctypes.data, sc.ctypes.data, c.ctypes.data,
-                                              b["tiles"].host(np.uint8)[off:].ctypes.data, b["max_tiles"])
-        if n == 0:
-            raise OmegaGpuError(-1, f"tile table larger than its region of {b['max_tiles']} entries")
-        return b["tiles"].va + off, n
+    def _put_dense(self, b, m):
+        """the tile tables of m rows over every layer's q|k|v and o weights, [layer][q|k|v, o][tile]"""
+        nt = -(-m // self.bm)
+        tab = np.zeros((len(self.layers), 2, nt), TILE_DTYPE)
+        for j, name in enumerate(("qkv", "o")):
+            tab["w_va"][:, j] = np.array([L["ent"][name][0] for L in self.layers])
+            tab["s_va"][:, j] = np.array([L["ent"][name][1] for L in self.layers])
+        tab["row0"] = self.bm * np.arange(nt)
+        tab["cnt"] = np.minimum(self.bm, m - self.bm * np.arange(nt))
+        self._up(b["dense"], tab)
+        return nt
+
+    def _put_plan(self, b, m, ent):
+        """Routes the m token rows of the staged logits (omega_gpu_pf_moe_plan) and moves the layer's
+        plan to the device. Returns the plan (views of the staging buffer: ids, weights, a2g) and its
+        tile count."""
+        e, top_k, at = self.e, self.top_k, b["plan_at"]
+        stage = b["stage"].host(np.uint8)
+        addr = [b["stage"].mem.cpu + b["plan_stage"] + v for v in at]
+        ids, counts = np.empty((m, top_k), np.uint32), np.empty(e, np.uint32)
+        _pf_check(lib().omega_gpu_pf_moe_plan(m, e, top_k, b["stage"].mem.cpu, ids.ctypes.data, addr[2],
+                                              counts.ctypes.data, addr[0], addr[1], None), "pf moe plan")
+        n = 0
+        for off, (w, sc) in ((3, ent["gu"]), (4, ent["dn"])):
+            n = lib().omega_gpu_pf_qgemm_tiles_va(e, w.ctypes.data, sc.ctypes.data, counts.ctypes.data, addr[off],
+                                                  b["max_tiles"])
+            if n == 0:
+                raise OmegaGpuError(-1, f"tile table larger than its region of {b['max_tiles']} entries")
+        copy_va(b["plan"].va, b["stage"].va + b["plan_stage"], at[-1])
+        g = m * top_k
+        view = lambda i, dt: stage[b["plan_stage"] + at[i]:b["plan_stage"] + at[i] + 4 * g].view(dt)
+        return ids, view(2, np.float32).reshape(m, top_k), view(1, np.uint32), n
 
     def run(self, tokens, pos0, trace=None):
         """Tokens at positions pos0 .. pos0 + m - 1 through every layer; returns the last token's
@@ -365,58 +398,56 @@ class WholePromptPrefill:
         h, qd, qkv_n, e, top_k, i, eps = self.h, self.qd, self.qkv_n, self.e, self.top_k, self.i, self.eps
         g = m * top_k
         b = self._ensure(m)
-        self._up(b["x"], np.stack([np.asarray(self.embed_row(t), np.float32) for t in tokens]))
+        rows = b["stage"].host(np.float32)[:m * h]
+        np.concatenate([np.asarray(self.embed_row(t), np.float32).reshape(-1) for t in tokens], out=rows)
+        copy_va(b["x"].va, b["stage"].va, (m * h * 4 + 15) // 16 * 16)
+        dense = self._put_dense(b, m)
         chip = 0
-        dense = [m]
         add = 0  # the previous layer's MoE rows, added to the residual by the next norm
         for l, L in enumerate(self.layers):
             ent = L["ent"]
             chip += residual_norm(h, m, b["x"].va, add, L["input_norm"].va, eps, b["xin"].va)
             if trace is not None and l > 0:
-                trace.setdefault("x_out", []).append(self._down(b["x"], np.float32, m * h).reshape(m, h))
+                trace.setdefault("x_out", []).append(self._down(b["x"], np.float32, m * h).reshape(m, h).copy())
             chip += quant(h, IN_F32, m, b["xin"].va, b["xq"].va, b["xs"].va)
-            tv, nt = self._put_tiles(b, 0, ent["qkv"], dense)
-            chip += qgemm(qkv_n, h, PLAIN, tv, nt, 0, b["xq"].va, b["xs"].va, b["qkv"].va)
+            tv = b["dense"].va + 2 * l * dense * TILE_BYTES
+            chip += qgemm(qkv_n, h, PLAIN, tv, dense, 0, b["xq"].va, b["xs"].va, b["qkv"].va)
             info = self.attn.attend_dev(l, pos0, m, b["qkv"].va, eps, 1.0, b["att"].va)
             chip += info.elapsed_ns
             if trace is not None:
-                trace.setdefault("qkv", []).append(self._down(b["qkv"], np.float32, m * qkv_n).reshape(m, qkv_n))
-                trace.setdefault("att", []).append(self._down(b["att"], np.float32, m * qd).reshape(m, qd))
+                trace.setdefault("qkv", []).append(self._down(b["qkv"], np.float32, m * qkv_n).reshape(m, qkv_n).copy())
+                trace.setdefault("att", []).append(self._down(b["att"], np.float32, m * qd).reshape(m, qd).copy())
             chip += quant(qd, IN_F32, m, b["att"].va, b["xq"].va, b["xs"].va)
-            tv, nt = self._put_tiles(b, 1, ent["o"], dense)
-            chip += qgemm(h, qd, PLAIN, tv, nt, 0, b["xq"].va, b["xs"].va, b["oproj"].va)
+            chip += qgemm(h, qd, PLAIN, tv + dense * TILE_BYTES, dense, 0, b["xq"].va, b["xs"].va, b["oproj"].va)
             # x += o_proj, then the post-norm rows: the quantiser's and the router's input
             chip += residual_norm(h, m, b["x"].va, b["oproj"].va, L["post_norm"].va, eps, b["xin"].va)
             chip += router_logits(h, e, m, b["xin"].va, L["wq"].va, b["logits"].va)
             logits = self._down(b["logits"], np.float32, m * e)
-            ids, wts, counts, grouped_token, a2g = moe_plan(logits, m, e, top_k)
             if trace is not None:
-                trace.setdefault("x_mid", []).append(self._down(b["x"], np.float32, m * h).reshape(m, h))
-                trace.setdefault("post", []).append(self._down(b["xin"], np.float32, m * h).reshape(m, h))
-                trace.setdefault("ids", []).append(ids.copy())
+                trace.setdefault("logits", []).append(logits.reshape(m, e).copy())
+            ids, wts, a2g, nt = self._put_plan(b, m, ent)
+            plan = [b["plan"].va + v for v in b["plan_at"]]
+            if trace is not None:
                 trace.setdefault("wts", []).append(wts.copy())
                 trace.setdefault("a2g", []).append(a2g.copy())
-                trace.setdefault("logits", []).append(logits.reshape(m, e).copy())
+                trace.setdefault("x_mid", []).append(self._down(b["x"], np.float32, m * h).reshape(m, h).copy())
+                trace.setdefault("post", []).append(self._down(b["xin"], np.float32, m * h).reshape(m, h).copy())
+                trace.setdefault("ids", []).append(ids.copy())
             chip += quant(h, IN_F32, m, b["xin"].va, b["xq"].va, b["xs"].va)
-            self._up(b["rowidx"], grouped_token)
-            tv, nt = self._put_tiles(b, 2, ent["gu"], counts)
-            chip += qgemm(2 * i, h, SWIGLU_NAT, tv, nt, b["rowidx"].va, b["xq"].va, b["xs"].va, b["act"].va)
+            chip += qgemm(2 * i, h, SWIGLU_NAT, plan[3], nt, plan[0], b["xq"].va, b["xs"].va, b["act"].va)
             chip += quant(i, IN_BF16, g, b["act"].va, b["aq"].va, b["a_s"].va)
-            tv, nt = self._put_tiles(b, 2, ent["dn"], counts)
-            chip += qgemm(h, i, PLAIN, tv, nt, 0, b["aq"].va, b["a_s"].va, b["down"].va)
-            self._up(b["inv"], a2g)
-            self._up(b["wts"], wts.reshape(-1))
-            chip += moe_combine(h, top_k, m, b["down"].va, b["inv"].va, b["wts"].va, b["moe"].va)
+            chip += qgemm(h, i, PLAIN, plan[4], nt, 0, b["aq"].va, b["a_s"].va, b["down"].va)
+            chip += moe_combine(h, top_k, m, b["down"].va, plan[1], plan[2], b["moe"].va)
             if trace is not None:
-                trace.setdefault("act", []).append(self._down(b["act"], np.uint16, g * i).reshape(g, i))
-                trace.setdefault("down", []).append(self._down(b["down"], np.float32, g * h).reshape(g, h))
+                trace.setdefault("act", []).append(self._down(b["act"], np.uint16, g * i).reshape(g, i).copy())
+                trace.setdefault("down", []).append(self._down(b["down"], np.float32, g * h).reshape(g, h).copy())
             add = b["moe"].va
         # the last MoE add, then the final norm (over every row: one launch either way)
         chip += residual_norm(h, m, b["x"].va, add, self.final_dev.va, eps, b["xin"].va)
         if trace is not None:
-            trace.setdefault("x_out", []).append(self._down(b["x"], np.float32, m * h).reshape(m, h))
+            trace.setdefault("x_out", []).append(self._down(b["x"], np.float32, m * h).reshape(m, h).copy())
         self.stats = dict(tokens=m, chip_ns=chip)
-        return self._down(b["xin"], np.float32, m * h)[(m - 1) * h:].copy()
+        return self._down(b["xin"], np.float32, h, (m - 1) * h).copy()
 
     def free(self):
         self.bufs = None
