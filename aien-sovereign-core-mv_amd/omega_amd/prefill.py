@@ -382,8 +382,10 @@ class WholePromptPrefill:
                                                   b["max_tiles"])
             if n == 0:
                 raise OmegaGpuError(-1, f"tile table larger than its region of {b['max_tiles']} entries")
-        copy_va(b["plan"].va, b["stage"].va + b["plan_stage"], at[-1])
+        # row indices past the last row are read with a tile of bm rows and must name a row
         g = m * top_k
+        stage[b["plan_stage"] + 4 * g:b["plan_stage"] + 4 * (g + self.bm)] = 0
+        copy_va(b["plan"].va, b["stage"].va + b["plan_stage"], at[-1])
         view = lambda i, dt: stage[b["plan_stage"] + at[i]:b["plan_stage"] + at[i] + 4 * g].view(dt)
         return ids, view(2, np.float32).reshape(m, top_k), view(1, np.uint32), n
 
