@@ -39,59 +39,80 @@ constexpr uint32_t kPfBm = 64;  // activation rows per tile
 constexpr uint32_t kPfLayoutPlain = 0, kPfLayoutSwiglu = 2;
 
 // ------------------------------------------------------------------ quantiser
-// f32 -> e4m3 code, round to nearest even, saturating to +-448, on the f32 bits (no dependence on
-// the float mode registers): below 2^-6 the codes are the multiples of 2^-9, above it the three
-// mantissa bits round on the 20 dropped ones.
-__device__ __forceinline__ uint32_t e4m3_rne_sat(float f) {
-    const uint32_t b = __float_as_uint(f), s = (b >> 24) & 0x80u, a = b & 0x7fffffffu;
-    if (a > 0x43e00000u) return s | 0x7eu;  // above 448 (and infinities)
-    if (a < 0x3c800000u) return s | (uint32_t)rintf(__uint_as_float(a) * 512.0f);
-    uint32_t e = (a >> 23) - 120u, m = (a >> 20) & 7u;
-    const uint32_t rem = a & 0xfffffu;
-    if (rem > 0x80000u || (rem == 0x80000u && (m & 1u))) {
-        if (++m == 8u) {
-            m = 0;
-            ++e;
-        }
-    }
-    const uint32_t code = (e << 3) | m;
-    return s | (code > 0x7eu ? 0x7eu : code);
-}
-
 struct PfQuantArgs {
-    uint32_t k = 0, rows = 0, bf16_in = 0;
+    uint32_t k = 0, rows = 0;
     const void *x = nullptr;
     uint8_t *q = nullptr;  // [rows][k]
     float *s = nullptr;    // [rows][k / 128]
 };
 
-// one wavefront per (row, 128-block): lane l holds values 2 l, 2 l + 1
+// e4m3 codes of two values already scaled into +-448 (beyond it, and NaN: the largest code of the
+// value's sign), round to nearest even
+template <bool HI>
+__device__ __forceinline__ int e4m3_pair(float a, float b, int old) {
+    auto sat = [](float f) {
+        const uint32_t u = __float_as_uint(f);
+        return __uint_as_float((u & 0x80000000u) | min(u & 0x7fffffffu, 0x43e00000u));
+    };
+    return __builtin_amdgcn_cvt_pk_fp8_f32(sat(a), sat(b), old, HI);
+}
+
+// A 128-block per 128 / V lanes, V consecutive values a lane; the blocks of all rows are one list.
+// V 8 (16 lanes, 16-byte loads, 8-byte stores, the block maximum inside a 16-lane row) is the form
+// for 16-byte aligned rows, V 2 (one wavefront a block) for other addresses. Bound by its bytes
+// through HBM and L2. Launch times, V 2 for everything before: 16000 rows of 768 bf16 values 22.8 ->
+// 8.7 us (4.2 TB/s), 2000 rows of 2048 f32 values 10.3 -> 6.6 us, an empty launch being 6.
+template <bool BF16, int V>
 __global__ __launch_bounds__(256) void k_pf_quant(const PfQuantArgs a) {
-    const uint32_t blocks = a.k / 128;
-    const uint32_t item = blockIdx.x * 4 + (threadIdx.x >> 6), lane = lane_id();
-    if (item >= a.rows * blocks) return;
-    const uint32_t row = item / blocks, b = item % blocks;
-    const size_t at = (size_t)row * a.k + 128 * b + 2 * lane;
-    float v0, v1;
-    if (a.bf16_in) {
-        const uint32_t w = *as_global_u32(static_cast<const uint16_t *>(a.x) + at);
-        v0 = __uint_as_float(w << 16);
-        v1 = __uint_as_float(w & 0xffff0000u);
+    constexpr uint32_t kLanes = 128 / V;
+    const uint64_t item = (uint64_t)blockIdx.x * (256 / kLanes) + threadIdx.x / kLanes;
+    if (item >= (uint64_t)a.rows * (a.k / 128)) return;
+    const uint32_t l = threadIdx.x % kLanes;
+    const size_t at = (size_t)item * 128 + V * l;
+    float v[V];
+    if constexpr (BF16) {
+        uint32_t w[V / 2];
+        const uint16_t *x = static_cast<const uint16_t *>(a.x) + at;
+        if constexpr (V == 8) {
+            const u32x4 t = *as_global(x);
+            w[0] = t.x, w[1] = t.y, w[2] = t.z, w[3] = t.w;
+        } else {
+            w[0] = *as_global_u32(x);
+        }
+#pragma unroll
+        for (int i = 0; i < V / 2; ++i) {
+            v[2 * i] = __uint_as_float(w[i] << 16);
+            v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+        }
     } else {
-        const u32x2 w = *as_global_u32x2(static_cast<const float *>(a.x) + at);
-        v0 = __uint_as_float(w.x);
-        v1 = __uint_as_float(w.y);
+        const float *x = static_cast<const float *>(a.x) + at;
+        if constexpr (V == 8) {
+            const f32x4 t = *as_global_f32x4(x), u = *as_global_f32x4(x + 4);
+            v[0] = t.x, v[1] = t.y, v[2] = t.z, v[3] = t.w, v[4] = u.x, v[5] = u.y, v[6] = u.z, v[7] = u.w;
+        } else {
+            const u32x2 t = *as_global_u32x2(x);
+            v[0] = __uint_as_float(t.x), v[1] = __uint_as_float(t.y);
+        }
     }
-    float m = fmaxf(fabsf(v0), fabsf(v1));
+    float m = fabsf(v[0]);
+#pragma unroll
+    for (int i = 1; i < V; ++i) m = fmaxf(m, fabsf(v[i]));
     m = row16_max(m);
-    m = fmaxf(fmaxf(readlane_f32(m, 0), readlane_f32(m, 16)), fmaxf(readlane_f32(m, 32), readlane_f32(m, 48)));
+    if constexpr (V == 2)
+        m = fmaxf(fmaxf(readlane_f32(m, 0), readlane_f32(m, 16)), fmaxf(readlane_f32(m, 32), readlane_f32(m, 48)));
     m = fmaxf(m, 7.888609052210118e-31f);  // 2^-100
     // scale 2^(E - 8), or 2^(E - 7) when the mantissa is above 1.75 (E the exponent of m)
     const uint32_t mb = __float_as_uint(m), e = mb >> 23, c = ((mb & 0x7fffffu) + 0x1fffffu) >> 23;
     const float scale = __uint_as_float((e + c - 8u) << 23), inv = __uint_as_float((262u - e - c) << 23);
-    const uint32_t q = e4m3_rne_sat(v0 * inv) | (e4m3_rne_sat(v1 * inv) << 8);
-    *reinterpret_cast<uint16_t *>(a.q + at) = (uint16_t)q;
-    if (lane == 0) a.s[(size_t)row * blocks + b] = scale;
+    if constexpr (V == 8) {
+        u32x2 q;
+        q.x = (uint32_t)e4m3_pair<true>(v[2] * inv, v[3] * inv, e4m3_pair<false>(v[0] * inv, v[1] * inv, 0));
+        q.y = (uint32_t)e4m3_pair<true>(v[6] * inv, v[7] * inv, e4m3_pair<false>(v[4] * inv, v[5] * inv, 0));
+        *reinterpret_cast<u32x2 *>(a.q + at) = q;
+    } else {
+        *reinterpret_cast<uint16_t *>(a.q + at) = (uint16_t)e4m3_pair<false>(v[0] * inv, v[1] * inv, 0);
+    }
+    if (l == 0) a.s[item] = scale;
 }
 
 // ------------------------------------------------------------------ grouped W8A8 GEMM
@@ -680,7 +701,6 @@ int omega_gpu_pf_quant(uint32_t k, uint32_t in_type, uint32_t rows, uint64_t x_v
     PfQuantArgs a;
     a.k = k;
     a.rows = rows;
-    a.bf16_in = in_type;
     a.x = (const void *)(uintptr_t)x_va;
     a.q = (uint8_t *)(uintptr_t)q_va;
     a.s = (float *)(uintptr_t)s_va;
@@ -690,7 +710,12 @@ int omega_gpu_pf_quant(uint32_t k, uint32_t in_type, uint32_t rows, uint64_t x_v
         return OMEGA_GPU_TOO_LARGE;
     }
     return pf_timed(F_SESSION, 1, ns, [&](hipStream_t st) {
-        OMEGA_LAUNCH(k_pf_quant, dim3((uint32_t)((waves + 3) / 4)), dim3(256), 0, st, a);
+        const dim3 wg(256), blocks4((uint32_t)((waves + 3) / 4)), blocks16((uint32_t)((waves + 15) / 16));
+        if (x_va % 16 || q_va % 8) {
+            if (in_type) OMEGA_LAUNCH((k_pf_quant<true, 2>), blocks4, wg, 0, st, a);
+            else OMEGA_LAUNCH((k_pf_quant<false, 2>), blocks4, wg, 0, st, a);
+        } else if (in_type) OMEGA_LAUNCH((k_pf_quant<true, 8>), blocks16, wg, 0, st, a);
+        else OMEGA_LAUNCH((k_pf_quant<false, 8>), blocks16, wg, 0, st, a);
         return hipGetLastError();
     });
 }

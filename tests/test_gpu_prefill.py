@@ -88,6 +88,30 @@ def test_quant_bf16_input_and_wide_rows(omega, oracle, pf):
         np.testing.assert_array_equal(q2[r], wq)
 
 
+@pytest.mark.parametrize("off", [0, 8])          # 16-byte aligned rows, and rows that are not
+@pytest.mark.parametrize("rows,k", [(1, 128), (15, 128), (17, 128), (3, 2176), (257, 768)])
+def test_quant_row_edges(omega, oracle, pf, rows, k, off):
+    rng = np.random.default_rng(rows + k)
+    x = (rng.standard_normal((rows, k)) * np.exp(rng.uniform(-8, 8, (rows, k)))).astype(np.float32)
+    x[:, 5] = 1.75 * np.ldexp(1.0, rng.integers(-3, 12, rows))  # often a block's largest value, on the scale's tie
+    x[0, 3], x[-1, -1] = np.inf, -0.0
+    for in_type, rowsin in ((pf.IN_F32, x), (pf.IN_BF16, oracle.f32_to_bf16(x))):
+        size = rowsin.dtype.itemsize
+        xd = dev_from(omega, np.concatenate([np.zeros(off // size, rowsin.dtype), rowsin.reshape(-1)]))
+        qd, sd = dev_from(omega, np.full(rows * k + 16, 0x55, np.uint8)), omega.DeviceBuffer(rows * k // 32)
+        pf.quant(k, in_type, rows, xd.ptr.value + off, qd.ptr.value + off, sd.ptr)
+        q, s = qd.download(np.uint8, rows * k + 16), sd.download(np.float32, rows * k // 128).reshape(rows, -1)
+        assert (q[:off] == 0x55).all() and (q[off + rows * k:] == 0x55).all()
+        q = q[off:off + rows * k].reshape(rows, k)
+        wide = oracle.bf16_to_f32(rowsin) if in_type == pf.IN_BF16 else rowsin
+        for r in range(rows):
+            first = 128 if r == 0 else 0  # the block with the infinity: its largest code, no defined others
+            wq, ws = oracle.quant_row(wide[r])
+            np.testing.assert_array_equal(q[r, first:], wq[first:])
+            np.testing.assert_array_equal(s[r, first // 128:].view(np.uint32), ws[first // 128:].view(np.uint32))
+        assert q[0, 3] == 0x7e
+
+
 def dequant_rows(oracle, q, s):
     t = oracle.e4m3_table()
     v = t[q].astype(np.float64)
