@@ -431,7 +431,11 @@ __global__ __launch_bounds__(256) void k_pf_router(const PfRouterArgs a) {
 
 // ------------------------------------------------------------------ MoE combine
 // out[r][c] = sum over slots in order, from +0.0, of wt[r][slot] * down[inv[r][slot]][c] (each
-// product rounded, then added). One thread per (row, column).
+// product rounded, then added). Bound by the top_k down rows it reads: one thread per row and V
+// columns (4 where h and the addresses allow 16-byte loads, else 1), the loads of 8 slots in flight
+// before the first is summed. The slots' rows and weights are the same for a whole workgroup and
+// come through scalar loads. Launch times, one column a thread and one slot in flight before: 2000
+// tokens of 8 x 2048 values 31.5 -> 24.7 us (6 TB/s), 517 tokens 12.4 -> 7.7 us.
 struct PfCombineArgs {
     uint32_t h = 0, top_k = 0, rows = 0;
     const float *down = nullptr;
@@ -440,17 +444,43 @@ struct PfCombineArgs {
     float *out = nullptr;
 };
 
+template <int V>
 __global__ __launch_bounds__(256) void k_pf_combine(const PfCombineArgs a) {
 #pragma clang fp contract(off)  // a multiply then an add, never one fused rounding
-    const uint32_t r = blockIdx.y, c = blockIdx.x * 256 + threadIdx.x;
+    const uint32_t r = blockIdx.y, c = (blockIdx.x * 256 + threadIdx.x) * V;
     if (c >= a.h) return;
-    float acc = 0.0f;
-    for (uint32_t s = 0; s < a.top_k; ++s) {
-        const uint32_t src = *as_global_u32(a.inv + (size_t)r * a.top_k + s);
-        const float w = *as_global_f32(a.wt + (size_t)r * a.top_k + s);
-        acc = acc + w * *as_global_f32(a.down + (size_t)src * a.h + c);
+    const cu32 *inv = as_const_u32(a.inv + (size_t)r * a.top_k), *wt = as_const_u32(a.wt + (size_t)r * a.top_k);
+    float acc[V] = {};
+    uint32_t s = 0;
+    auto load = [&](uint32_t slot, float (&d)[V]) {
+        const float *p = a.down + (size_t)inv[slot] * a.h + c;
+        if constexpr (V == 4) {
+            const f32x4 t = *as_global_f32x4(p);
+            d[0] = t.x, d[1] = t.y, d[2] = t.z, d[3] = t.w;
+        } else {
+            d[0] = *as_global_f32(p);
+        }
+    };
+    auto add = [&](uint32_t slot, const float (&d)[V]) {
+        const float w = __uint_as_float(wt[slot]);
+#pragma unroll
+        for (int i = 0; i < V; ++i) acc[i] = acc[i] + w * d[i];
+    };
+    for (; s + 8 <= a.top_k; s += 8) {
+        float d[8][V];
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) load(s + j, d[j]);
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) add(s + j, d[j]);
     }
-    a.out[(size_t)r * a.h + c] = acc;
+    for (; s < a.top_k; ++s) {
+        float d[V];
+        load(s, d);
+        add(s, d);
+    }
+    float *o = a.out + (size_t)r * a.h + c;
+    if constexpr (V == 4) *reinterpret_cast<f32x4 *>(o) = f32x4{acc[0], acc[1], acc[2], acc[3]};
+    else o[0] = acc[0];
 }
 
 // ------------------------------------------------------------------ residual add + RMSNorm (extension)
@@ -971,7 +1001,10 @@ int omega_gpu_pf_moe_combine(uint32_t h, uint32_t top_k, uint32_t rows, uint64_t
     a.wt = reinterpret_cast<const float *>(wt_va);
     a.out = reinterpret_cast<float *>(out_va);
     return pf_timed(F_SESSION, 1, ns, [&](hipStream_t st) {
-        OMEGA_LAUNCH(k_pf_combine, dim3((h + 255) / 256, rows), dim3(256), 0, st, a);
+        if (h % 4 == 0 && down_va % 16 == 0 && out_va % 16 == 0)
+            OMEGA_LAUNCH(k_pf_combine<4>, dim3((h + 1023) / 1024, rows), dim3(256), 0, st, a);
+        else
+            OMEGA_LAUNCH(k_pf_combine<1>, dim3((h + 255) / 256, rows), dim3(256), 0, st, a);
         return hipGetLastError();
     });
 }

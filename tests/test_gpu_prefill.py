@@ -265,9 +265,9 @@ def test_router_logits_are_the_sequential_f32_sum(omega, oracle, pf, e, k, rows)
     np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
-def test_moe_combine_slot_order(omega, pf):
+@pytest.mark.parametrize("h,top_k,rows", [(2048, 8, 13), (4, 1, 3), (1028, 9, 5), (1023, 8, 2), (257, 17, 4)])
+def test_moe_combine_slot_order(omega, pf, h, top_k, rows):
     rng = np.random.default_rng(7)
-    h, top_k, rows = 2048, 8, 13
     g = rows * top_k
     down = rng.standard_normal((g, h)).astype(np.float32)
     inv = rng.permutation(g).astype(np.uint32)
