@@ -495,27 +495,60 @@ struct PfNormArgs {
     float *out = nullptr;
 };
 
+// One workgroup per row, thread t takes columns t, t + 256, ... NV > 0 (rows of up to 256 NV
+// columns): all of a thread's columns are loaded before the first is used and stay in registers
+// until the normalised row is written. NV 0 (longer rows) walks them one by one and reads the row
+// again for the output. The sums have one order in both. Launch times, NV 0 for everything before: 517
+// rows of 2048 with an addend 8.8 -> 7.0 us, 2000 rows 14.7 -> 11.6 us (5.6 TB/s).
+template <int NV>
 __global__ __launch_bounds__(256) void k_pf_resid_norm(const PfNormArgs a) {
 #pragma clang fp contract(off)  // x + add and x * scale * w each rounded as written
     __shared__ double red[4];
     const uint32_t r = blockIdx.x, t = threadIdx.x, lane = lane_id(), wid = t >> 6;
     float *xr = a.x + (size_t)r * a.k;
     const float *ar = a.add ? a.add + (size_t)r * a.k : nullptr;
+    float *orow = a.out + (size_t)r * a.k;
+    float v[NV ? NV : 1], w[NV ? NV : 1], d[NV ? NV : 1];
     double ss = 0.0;
-    for (uint32_t c = t; c < a.k; c += 256) {
-        float v = xr[c];
-        if (ar) {
-            v = v + ar[c];
-            xr[c] = v;
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (uint32_t i = 0; i < NV; ++i) {
+            const uint32_t c = min(t + 256 * i, a.k - 1);  // lanes past the end read the last column
+            v[i] = *as_global_f32(xr + c);
+            w[i] = *as_global_f32(a.w + c);
+            d[i] = ar ? *as_global_f32(ar + c) : 0.f;
         }
-        ss += (double)v * (double)v;
+#pragma unroll
+        for (uint32_t i = 0; i < NV; ++i) {
+            const uint32_t c = t + 256 * i;
+            if (c >= a.k) continue;
+            if (ar) {
+                v[i] = v[i] + d[i];
+                xr[c] = v[i];
+            }
+            ss += (double)v[i] * (double)v[i];
+        }
+    } else {
+        for (uint32_t c = t; c < a.k; c += 256) {
+            float x = xr[c];
+            if (ar) {
+                x = x + ar[c];
+                xr[c] = x;
+            }
+            ss += (double)x * (double)x;
+        }
     }
     ss = wave_sum_f64(ss);
     if (lane == 0) red[wid] = ss;
     __syncthreads();
     const float scale = rms_scale((red[0] + red[1]) + (red[2] + red[3]), a.k, a.eps);
-    float *orow = a.out + (size_t)r * a.k;
-    for (uint32_t c = t; c < a.k; c += 256) orow[c] = xr[c] * scale * a.w[c];
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (uint32_t i = 0; i < NV; ++i)
+            if (t + 256 * i < a.k) orow[t + 256 * i] = v[i] * scale * w[i];
+    } else {
+        for (uint32_t c = t; c < a.k; c += 256) orow[c] = xr[c] * scale * a.w[c];
+    }
 }
 
 // ------------------------------------------------------------------ host threads for per-token host work
@@ -1027,7 +1060,9 @@ int omega_gpu_pf_residual_norm(uint32_t k, uint32_t rows, uint64_t x_va, uint64_
     a.eps = eps;
     a.out = reinterpret_cast<float *>(out_va);
     return pf_timed(F_SESSION, 1, ns, [&](hipStream_t st) {
-        OMEGA_LAUNCH(k_pf_resid_norm, dim3(rows), dim3(256), 0, st, a);
+        if (k <= 256 * 8) OMEGA_LAUNCH(k_pf_resid_norm<8>, dim3(rows), dim3(256), 0, st, a);
+        else if (k <= 256 * 16) OMEGA_LAUNCH(k_pf_resid_norm<16>, dim3(rows), dim3(256), 0, st, a);
+        else OMEGA_LAUNCH(k_pf_resid_norm<0>, dim3(rows), dim3(256), 0, st, a);
         return hipGetLastError();
     });
 }

@@ -285,6 +285,29 @@ def test_moe_combine_slot_order(omega, pf, h, top_k, rows):
     np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("k,rows,off", [
+    (4, 3, 0), (1020, 2, 0), (1024, 2, 0), (1028, 5, 0), (2048, 7, 0), (3000, 2, 0), (4096, 3, 0),  # in registers
+    (4100, 2, 0), (8192, 1, 0), (101, 3, 0), (2048, 3, 4),                                          # the general form
+])
+def test_residual_norm_row_edges(omega, pf, k, rows, off):
+    rng = np.random.default_rng(k + rows)
+    x, add = rng.standard_normal((2, rows, k)).astype(np.float32)
+    w = (1 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    pad = np.full(off // 4, 7.0, np.float32)
+    for given in (False, True):
+        xd, ad, wd = (dev_from(omega, np.concatenate([pad, v.reshape(-1), pad])) for v in (x, add, w))
+        od = dev_from(omega, np.full(rows * k + 8, 7.0, np.float32))
+        pf.residual_norm(k, rows, xd.ptr.value + off, ad.ptr.value + off if given else 0, wd.ptr.value + off, 1e-6, od.ptr.value + off)
+        xn = x + add if given else x
+        np.testing.assert_array_equal(xd.download(np.float32, rows * k + off // 4)[off // 4:].reshape(rows, k), xn)
+        got = od.download(np.float32, rows * k + 8)
+        assert (got[:off // 4] == 7.0).all() and (got[off // 4 + rows * k:] == 7.0).all()
+        x64 = xn.astype(np.float64)
+        want = x64 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + 1e-6) * w
+        # three f32 roundings (the scale, x * scale, * w) of 2^-24 each, beside the sum's in 64 bits
+        np.testing.assert_allclose(got[off // 4:off // 4 + rows * k].reshape(rows, k), want, rtol=4 * 2.0 ** -24)
+
+
 @pytest.mark.parametrize("N,first", [(300, 100), (1300, 1030)])
 def test_prefill_attention_equals_the_decode_attention(omega, oracle, pf, N, first):
     # (1300, 1030): contexts past 1024 take the 4-token query tiles, the first call spans two
