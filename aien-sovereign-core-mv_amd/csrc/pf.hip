@@ -21,6 +21,8 @@
 #include <functional>
 #include <mutex>
 #include <thread>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 #include <pthread.h>
@@ -346,16 +348,25 @@ __global__ __launch_bounds__(PAIR ? 512 : 256, PAIR ? 2 : 3) void k_pf_qgemm(con
 // logits[r][ex] = (((-0.0 + w[ex][0] x[r][0]) + w[ex][1] x[r][1]) + ...): each product rounded to
 // f32, then added in index order (no fused multiply-add), the reference's sequential f32 sum. The
 // sum cannot be split along k, so the parallelism is (row, expert): one lane per expert, R rows
-// per lane as R independent chains. The packed layout wq[g][ex][q] = w[ex][4 g + q] gives a
-// wavefront of 64 experts one contiguous KiB per group of 4 columns; the R rows of x are staged
-// through LDS in passes of kPfRouterKc columns and read as broadcasts, and the weight groups are
-// loaded kPfRouterNg at a time in two register sets so the next set is in flight while one is
-// summed. Rows come in tiles of kPfRouterRows (the buffers hold whole tiles): 16, the reference
-// engine's rows per CTA that the reference's own tests expect of router_rows()
-// (aien-omega-pf/src/lib.rs:1300); a launch takes 4, 2 or 1 rows per lane of such tiles.
+// per lane as R independent chains. Rows come in tiles of kPfRouterRows (the buffers hold whole
+// tiles): 16, the reference engine's rows per CTA that the reference's own tests expect of
+// router_rows() (aien-omega-pf/src/lib.rs:1300).
+//
+// A workgroup is 64 experts x 4 wavefronts of R rows each. The packed layout
+// wq[g][ex][q] = w[ex][4 g + q] gives 64 experts one contiguous KiB per group of 4 columns; the
+// weights come in passes of kPfRouterG groups, loaded by all four wavefronts into registers
+// kPfRouterAhead passes ahead and handed over through two LDS buffers with one barrier a pass. What
+// bounds it otherwise is the weight stream into the CUs (about 20 bytes a clock each): a wavefront
+// that reads the weights by itself takes 4 times as many. The x values of a pass
+// sit in registers, 16 columns each in every 16-lane row, and reach the product as its DPP row
+// broadcast, so they cost no LDS reads and no instructions. What is left is the chain: a product and
+// a sum per column, 25 us for 2048 columns with one wavefront a SIMD and one row a lane.
+// Launch times against a wavefront that reads weights and x values by itself, 128 experts: 17 rows
+// 27.8 -> 24.7 us, 517 rows 31.3 -> 30.5 (behind the layer's other kernels 40.6 -> 31), 1024 rows
+// 49.3 -> 35.5, 2048 rows 92.5 -> 54.6, 4096 rows 96.0 -> 84.8 us.
 constexpr uint32_t kPfRouterRows = 16;
-constexpr uint32_t kPfRouterKc = 1024;
-constexpr uint32_t kPfRouterNg = 4;
+constexpr uint32_t kPfRouterG = 16;
+constexpr uint32_t kPfRouterAhead = 4;
 
 struct PfRouterArgs {
     uint32_t k = 0, e = 0, rows = 0;
@@ -363,65 +374,95 @@ struct PfRouterArgs {
     float *logits = nullptr;
 };
 
+// the value of lane N of the lane's 16-lane row
+template <int N>
+__device__ __forceinline__ float pf_row_bcast(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + N, 0xF, 0xF, true));
+}
+template <int... Q, class F>
+__device__ __forceinline__ void pf_for_each(std::integer_sequence<int, Q...>, F f) {
+    (f(std::integral_constant<int, Q>{}), ...);
+}
+
 template <int R>
 __global__ __launch_bounds__(256) void k_pf_router(const PfRouterArgs a) {
 #pragma clang fp contract(off)  // a multiply then an add, never one fused rounding
-    constexpr uint32_t NG = kPfRouterNg, KQ = kPfRouterKc / 4;
-    __shared__ f32x4 xs[R][KQ];
-    const uint32_t tid = threadIdx.x, nt = blockDim.x;
-    const uint32_t ex = blockIdx.x * nt + tid;
-    const uint32_t exl = ex < a.e ? ex : a.e - 1;  // lanes past the last expert load its weights
-    const uint32_t r0 = blockIdx.y * R;
-    const size_t gs = (size_t)a.e * 4;
-    const float *wp = a.wq + (size_t)exl * 4;
-    float acc[R];
+    constexpr uint32_t G = kPfRouterG, D = kPfRouterAhead;
+    __shared__ f32x4 L[2][G][64];
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t ex = blockIdx.x * 64 + lane, exl = min(ex, a.e - 1);  // lanes past the last expert load its weights
+    const uint32_t r0 = (blockIdx.y * 4 + wid) * R;
+    const uint32_t ng = a.k / 4, np = (ng + G - 1) / G, last = np - 1;
+    struct Set {
+        f32x4 w[G / 4];        // groups wid, wid + 4, ... of the pass
+        float x[R][G / 4];     // columns 16 i + lane % 16 of the pass
+    };
+    Set S[D];
+    auto load = [&](Set &s, uint32_t p) {
 #pragma unroll
-    for (int j = 0; j < R; ++j) acc[j] = -0.0f;
-    auto sum_group = [&](const f32x4 w, uint32_t q) {
+        for (uint32_t i = 0; i < G / 4; ++i) {  // past the last group and column: the last one again, unused
+            s.w[i] = *as_global_f32x4(a.wq + ((size_t)min(G * p + wid + 4 * i, ng - 1) * a.e + exl) * 4);
 #pragma unroll
-        for (int j = 0; j < R; ++j) {
-            const f32x4 xv = xs[j][q];
-            acc[j] = acc[j] + w.x * xv.x;
-            acc[j] = acc[j] + w.y * xv.y;
-            acc[j] = acc[j] + w.z * xv.z;
-            acc[j] = acc[j] + w.w * xv.w;
+            for (int j = 0; j < R; ++j)
+                s.x[j][i] = *as_global_f32(a.x + (size_t)(r0 + j) * a.k + min(4 * G * p + 16 * i + (lane & 15), a.k - 1));
         }
     };
-    const uint32_t ng = a.k / 4;
-    for (uint32_t c0 = 0; c0 < ng; c0 += KQ) {
-        const uint32_t cn = ng - c0 < KQ ? ng - c0 : KQ;  // groups in this pass
-        __syncthreads();                                  // the previous pass is read
-        for (uint32_t i = tid; i < R * cn; i += nt) {
-            const uint32_t j = i / cn, q = i - j * cn;
-            xs[j][q] = *as_global_f32x4(a.x + (size_t)(r0 + j) * a.k + 4 * (size_t)(c0 + q));
-        }
-        __syncthreads();
-        const float *wc = wp + (size_t)c0 * gs;
-        auto load = [&](f32x4 (&w)[NG], uint32_t q) {
+    float acc[R], xc[R][G / 4];
 #pragma unroll
-            for (uint32_t i = 0; i < NG; ++i) w[i] = *as_global_f32x4(wc + (size_t)(q + i) * gs);
-        };
-        auto sum_set = [&](const f32x4 (&w)[NG], uint32_t q) {
+    for (int j = 0; j < R; ++j) acc[j] = -0.0f;
+    // the pass's weights to LDS buffer b, its x values to xn
+    auto stage = [&](const Set &s, uint32_t b, float (&xn)[R][G / 4]) {
 #pragma unroll
-            for (uint32_t i = 0; i < NG; ++i) sum_group(w[i], q + i);
-        };
-        uint32_t q = 0;
-        if (cn >= 2 * NG) {
-            f32x4 A[NG], B[NG];
-            load(A, 0);
-            for (; q + 2 * NG <= cn; q += 2 * NG) {
-                load(B, q + NG);
-                sum_set(A, q);
-                const uint32_t qa = q + 2 * NG <= cn - NG ? q + 2 * NG : cn - NG;  // stays in the pass
-                load(A, qa);
-                sum_set(B, q + NG);
-            }
-            if (q + NG <= cn) {  // A holds the set at q
-                sum_set(A, q);
-                q += NG;
-            }
+        for (uint32_t i = 0; i < G / 4; ++i) {
+            L[b][wid + 4 * i][lane] = s.w[i];
+#pragma unroll
+            for (int j = 0; j < R; ++j) xn[j][i] = s.x[j][i];
         }
-        for (; q < cn; ++q) sum_group(*as_global_f32x4(wc + (size_t)q * gs), q);
+    };
+    auto group = [&](const f32x4 w, auto qc) {
+        constexpr int q = decltype(qc)::value, c = 4 * (q & 3);
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const float x = xc[j][q / 4], p0 = pf_row_bcast<c>(x) * w.x, p1 = pf_row_bcast<c + 1>(x) * w.y;
+            const float p2 = pf_row_bcast<c + 2>(x) * w.z, p3 = pf_row_bcast<c + 3>(x) * w.w;
+            acc[j] = acc[j] + p0;
+            acc[j] = acc[j] + p1;
+            acc[j] = acc[j] + p2;
+            acc[j] = acc[j] + p3;
+        }
+    };
+    // the first n groups of the pass in buffer b; all its LDS reads go out before the first sum
+    auto sums = [&](uint32_t b, uint32_t n, auto full) {
+        f32x4 w[G];
+#pragma unroll
+        for (uint32_t q = 0; q < G; ++q) w[q] = L[b][q][lane];
+        __builtin_amdgcn_sched_barrier(0);
+        pf_for_each(std::make_integer_sequence<int, (int)G>{}, [&](auto q) {
+            if (decltype(full)::value || q < n) group(w[q], q);
+        });
+    };
+#pragma unroll
+    for (uint32_t u = 0; u < D; ++u) load(S[u], min(u, last));
+    stage(S[0], 0, xc);
+    load(S[0], min(D, last));
+    lds_sync();
+    for (uint32_t p0 = 0; p0 < np; p0 += D) {
+#pragma unroll
+        for (uint32_t u = 0; u < D; ++u) {
+            const uint32_t p = p0 + u;
+            if (p >= np) break;  // the same for the whole workgroup
+            float xn[R][G / 4];
+            Set &s = S[(u + 1) % D];
+            stage(s, (u + 1) & 1, xn);
+            load(s, min(p + 1 + D, last));
+            if (G * (p + 1) <= ng) sums(u & 1, G, std::true_type{});
+            else sums(u & 1, ng - G * p, std::false_type{});
+            lds_sync();
+#pragma unroll
+            for (int j = 0; j < R; ++j)
+#pragma unroll
+                for (uint32_t i = 0; i < G / 4; ++i) xc[j][i] = xn[j][i];
+        }
     }
     if (ex < a.e) {
 #pragma unroll
@@ -986,12 +1027,11 @@ int omega_gpu_pf_router_logits(uint32_t k, uint32_t e, uint32_t rows, uint64_t x
     a.x = reinterpret_cast<const float *>(x_va);
     a.wq = reinterpret_cast<const float *>(wq_va);
     a.logits = reinterpret_cast<float *>(logits_va);
-    // a workgroup spans up to 256 experts; R rows per lane when that still gives one wavefront
-    // per SIMD (1024 on the chip), else fewer
-    const uint32_t waves_e = (e + 63) / 64, ew = waves_e < 4 ? waves_e : 4, nt = 64 * ew;
-    const uint32_t gx = (e + nt - 1) / nt;
-    const uint64_t waves1 = (uint64_t)gx * ew * a.rows;
-    const int r = waves1 >= 4 * 1024ull ? 4 : waves1 >= 2 * 1024ull ? 2 : 1;
+    // R rows per lane when that still gives every CU a workgroup, else fewer: a wavefront's four
+    // chains of 2048 columns take 55 us, its one chain 25 us
+    const uint32_t gx = (e + 63) / 64;
+    const uint64_t wgs = (uint64_t)gx * (a.rows / 4);
+    const int r = wgs >= 4 * 256ull ? 4 : wgs >= 2 * 256ull ? 2 : 1;
     const uint32_t max_rows = 32768 * (uint32_t)r;  // grid.y stays within 32768 row groups
     const uint32_t launches = (a.rows + max_rows - 1) / max_rows;
     return pf_timed(F_SESSION, launches, ns, [&](hipStream_t st) {
@@ -1000,13 +1040,13 @@ int omega_gpu_pf_router_logits(uint32_t k, uint32_t e, uint32_t rows, uint64_t x
             b.rows = a.rows - r0 < max_rows ? a.rows - r0 : max_rows;
             b.x = a.x + (size_t)r0 * k;
             b.logits = a.logits + (size_t)r0 * e;
-            const dim3 grid(gx, b.rows / r);
+            const dim3 grid(gx, b.rows / (4 * r));
             if (r == 4)
-                OMEGA_LAUNCH(k_pf_router<4>, grid, dim3(nt), 0, st, b);
+                OMEGA_LAUNCH(k_pf_router<4>, grid, dim3(256), 0, st, b);
             else if (r == 2)
-                OMEGA_LAUNCH(k_pf_router<2>, grid, dim3(nt), 0, st, b);
+                OMEGA_LAUNCH(k_pf_router<2>, grid, dim3(256), 0, st, b);
             else
-                OMEGA_LAUNCH(k_pf_router<1>, grid, dim3(nt), 0, st, b);
+                OMEGA_LAUNCH(k_pf_router<1>, grid, dim3(256), 0, st, b);
             const hipError_t err = hipGetLastError();
             if (err != hipSuccess) return err;
         }

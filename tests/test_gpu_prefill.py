@@ -241,7 +241,7 @@ def sequential_logits(wq_rows, x):
     return acc
 
 
-@pytest.mark.parametrize("e,k,rows", [(128, 2048, 9), (72, 100, 5), (300, 3000, 7), (128, 2048, 1100),
+@pytest.mark.parametrize("e,k,rows", [(1, 4, 1), (130, 260, 40), (65, 64, 1040), (128, 320, 2100), (128, 2048, 9), (72, 100, 5), (300, 3000, 7), (128, 2048, 1100),
                                       (128, 2048, 2049)])
 def test_router_logits_are_the_sequential_f32_sum(omega, oracle, pf, e, k, rows):
     # rows 1100 and 2049 take the 2- and 4-row-per-lane launches; e = 72 and 300 leave lanes
