@@ -362,7 +362,7 @@ __global__ __launch_bounds__(PAIR ? 512 : 256, PAIR ? 2 : 3) void k_pf_qgemm(con
 // broadcast, so they cost no LDS reads and no instructions. What is left is the chain: a product and
 // a sum per column, 25 us for 2048 columns with one wavefront a SIMD and one row a lane.
 // Launch times against a wavefront that reads weights and x values by itself, 128 experts: 17 rows
-// 27.8 -> 24.7 us, 517 rows 31.3 -> 30.5 (behind the layer's other kernels 40.6 -> 31), 1024 rows
+// 27.8 -> 24.7 us, 517 rows 31.3 -> 30.5 (behind the layer's other kernels 40.6 -> 29), 1024 rows
 // 49.3 -> 35.5, 2048 rows 92.5 -> 54.6, 4096 rows 96.0 -> 84.8 us.
 constexpr uint32_t kPfRouterRows = 16;
 constexpr uint32_t kPfRouterG = 16;
