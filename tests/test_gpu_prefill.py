@@ -205,6 +205,7 @@ def test_qgemm_grouped_swiglu_and_down(omega, oracle, pf):
     (128, 128, [1]),                                   # one k-block, one row
     (384, 384, [64, 1, 63]),                           # odd k-blocks, tiles at and beside 64 rows
     (256, 256, [17, 0, 65, 128]),
+    (256, 640, [31, 32, 33, 96, 97]),                  # tiles at and beside 32 rows, the short tiles' form
     # the paired form (256-row workgroups over two tiles of a run): runs of 1 to 5 tiles, full and
     # partial ends, so pairs start at even and at odd tiles of the table
     (512, 12288, [64, 128, 65, 1, 192, 320, 129, 63, 256, 200, 64, 300, 130, 640, 511]),
