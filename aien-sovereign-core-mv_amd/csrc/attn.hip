@@ -743,6 +743,20 @@ __device__ __forceinline__ void bf16_split_pair(float x, float y, uint32_t &hi, 
     lo = __builtin_bit_cast(uint32_t, l);
 }
 
+// kPattnC times a query's largest raw score so far, rounded: what every exponent of the query is taken
+// against (0 before the first key). The rounding must not be fused away where two of them meet: a
+// query whose maximum stays then has the factor 2^0, whatever its neighbours' rescaling.
+constexpr float kPattnC = kInvSqrt128 * 1.4426950408889634f;  // exp(s / sqrt 128) = 2^(kPattnC s)
+__device__ __forceinline__ float pattn_ref(float m) {
+#pragma clang fp contract(off)
+    return m == -INFINITY ? 0.f : m * kPattnC;
+}
+// 2^(from - to) for sums kept against the reference `from` that go over to `to`; nothing (0) where
+// no key was seen (m -inf)
+__device__ __forceinline__ float pattn_factor(float m, float from, float to) {
+    return m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(from - to);
+}
+
 // Eight wavefronts: qw = w % 4 owns 32 queries (4 tokens x 8 heads), kw = w / 4 takes every other
 // block of 32 keys; the two halves' states meet in LDS at the end. A block's K and V go through LDS
 // once for the four wavefronts of a half, one block ahead in registers, two LDS buffers, one barrier
@@ -858,8 +872,7 @@ __global__ __launch_bounds__(512, 2) void k_pattn(const PattnArgs a) {
     }
     lds_sync();  // the q rows are read
 
-    constexpr float kC = kInvSqrt128 * 1.4426950408889634f;      // exp(s / sqrt 128) = 2^(kC s)
-    float m_l = -INFINITY, l_l = 0.f;                            // l: this lane's keys only
+    float m_l = -INFINITY, ref = 0.f, l_l = 0.f;                 // ref: pattn_ref(m); l: this lane's keys only
     f32x16 O[4];                                                 // O[dt][i]: dim 32 dt + 8 (i / 4) + 4 hl + i % 4
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
@@ -889,24 +902,23 @@ __global__ __launch_bounds__(512, 2) void k_pattn(const PattnArgs a) {
         for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
         mx = xor_max<32>(mx);
         const float m_new = fmaxf(m_l, mx);
-        const float m_ref = m_new == -INFINITY ? 0.f : m_new;
-        const float mc = -m_ref * kC;
         if (__any(m_new != m_l)) {                               // else every factor is 1
-            const float alpha = __builtin_amdgcn_exp2f(fmaf(m_l, kC, mc));
+            const float to = pattn_ref(m_new), alpha = pattn_factor(m_l, ref, to);
             l_l *= alpha;
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) O[dt][i] *= alpha;
             m_l = m_new;
+            ref = to;
         }
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
             u32x4 hi, lo;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float p0 = __builtin_amdgcn_exp2f(fmaf(s[8 * kk + 2 * e], kC, mc));
-                const float p1 = __builtin_amdgcn_exp2f(fmaf(s[8 * kk + 2 * e + 1], kC, mc));
+                const float p0 = __builtin_amdgcn_exp2f(fmaf(s[8 * kk + 2 * e], kPattnC, -ref));
+                const float p1 = __builtin_amdgcn_exp2f(fmaf(s[8 * kk + 2 * e + 1], kPattnC, -ref));
                 l_l += p0 + p1;
                 uint32_t x, y;
                 bf16_split_pair(p0, p1, x, y);
@@ -946,9 +958,10 @@ __global__ __launch_bounds__(512, 2) void k_pattn(const PattnArgs a) {
     lds_sync();
     if (kw == 1) return;
     {
-        const float m1 = mls[0][qw][lane], M = fmaxf(m_l, m1), mc = M == -INFINITY ? 0.f : -M * kC;
-        const float w0 = __builtin_amdgcn_exp2f(fmaf(m_l, kC, mc)), w1 = __builtin_amdgcn_exp2f(fmaf(m1, kC, mc));
+        const float m1 = mls[0][qw][lane], M = fmaxf(m_l, m1), to = pattn_ref(M);
+        const float w0 = pattn_factor(m_l, ref, to), w1 = pattn_factor(m1, pattn_ref(m1), to);
         m_l = M;
+        ref = to;
         l_l = fmaf(l_l, w0, mls[1][qw][lane] * w1);
         l_l = xor_sum<32>(l_l);
 #pragma unroll
@@ -965,7 +978,7 @@ __global__ __launch_bounds__(512, 2) void k_pattn(const PattnArgs a) {
     } else {
         float *pp = a.part + (((size_t)(t0 + j) * a.nch + c) * 32 + h * 8 + head) * kPartStride;
         if (hl == 0) {
-            pp[0] = m_l * kInvSqrt128;
+            pp[0] = m_l == -INFINITY ? m_l : ref;
             pp[1] = l_l;
         }
         dst = pp + 4;
@@ -1426,15 +1439,11 @@ hipError_t launch_attn_combine(const CombineArgs &a, hipStream_t st) {
     return hipGetLastError();
 }
 
-// The items of every (seq, q head) combined, then split into the o projection's e4m3 terms (the
-// head's 128 dims are one 128-column block of o's input). Workgroup = (seq, head) of 256 threads:
-// the items' (m, l) are read by thread j % 256 of item j, their weights exp(m - M) staged in LDS;
-// thread t then sums dims 4 (t % 32) .. +3 over the items j = t / 32 (mod 8) and the 8 groups
-// meet in LDS in a fixed order; 16 lanes split the head's row.
 // The f32 rows of sequences (prefill tokens) of nch <= 64 partials each: one wavefront per (sequence,
-// q head), lane j holding partial j's (m, l), lane l dims l and l + 64; the partials
-// merge in item order (out = sum w_j o_j / sum w_j l_j with w_j = exp(m_j - max m), times
-// out_scale). A token always has a partial that sees its own position, so the maximum is finite.
+// q head), lane j holding partial j's (m, l), m in powers of two (k_pattn's reference, -inf where no
+// key was seen), lane l dims l and l + 64; the partials merge in item order (out = sum w_j o_j /
+// sum w_j l_j with w_j = 2^(m_j - max m), times out_scale). A token always has a partial that sees
+// its own position, so the maximum is finite.
 __global__ __launch_bounds__(256) void k_attn_combine_rows(const CombineItemsArgs a, uint32_t seqs, uint32_t nch) {
     const uint32_t lane = lane_id(), wv = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (wv >= seqs * 32) return;  // uniform per wavefront
@@ -1446,7 +1455,7 @@ __global__ __launch_bounds__(256) void k_attn_combine_rows(const CombineItemsArg
     const float mj = lane < n ? __uint_as_float(ml.x) : -INFINITY;
     float M = row16_max(mj);
     M = fmaxf(fmaxf(readlane_f32(M, 0), readlane_f32(M, 16)), fmaxf(readlane_f32(M, 32), readlane_f32(M, 48)));
-    const float wj = lane < n ? expf(mj - M) : 0.f;
+    const float wj = lane < n ? __builtin_amdgcn_exp2f(mj - M) : 0.f;
     const float L = wave_sum(wj * (lane < n ? __uint_as_float(ml.y) : 0.f));
     float o0 = 0.f, o1 = 0.f;
     for (uint32_t i = 0; i < n; ++i) {
@@ -1460,6 +1469,11 @@ __global__ __launch_bounds__(256) void k_attn_combine_rows(const CombineItemsArg
     out[64 + lane] = o1 / L * a.out_scale;
 }
 
+// The items of every (seq, q head) combined, then split into the o projection's e4m3 terms (the
+// head's 128 dims are one 128-column block of o's input). Workgroup = (seq, head) of 256 threads:
+// the items' (m, l) are read by thread j % 256 of item j, their weights exp(m - M) staged in LDS;
+// thread t then sums dims 4 (t % 32) .. +3 over the items j = t / 32 (mod 8) and the 8 groups
+// meet in LDS in a fixed order; 16 lanes split the head's row.
 __global__ __launch_bounds__(256) void k_attn_combine_items(const CombineItemsArgs a) {
     constexpr uint32_t kRounds = (kCombineMaxItems + 255) / 256;
     __shared__ float wsh[kRounds * 256];

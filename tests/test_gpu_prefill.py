@@ -395,6 +395,60 @@ def test_prefill_attention_tile_edges(omega, oracle, pf, pos0, m):
     c.free()
 
 
+def rot(x, pos, theta=1e6):
+    """x [..][128] rotated by RoPE at pos (rotate_half pairs i, i + 64), f64; -pos undoes it"""
+    ang = pos * theta ** (-np.arange(64) / 64.0)
+    a, b = x[..., :64], x[..., 64:]
+    return np.concatenate([a * np.cos(ang) - b * np.sin(ang), b * np.cos(ang) + a * np.sin(ang)], -1)
+
+
+def test_prefill_attention_rescale_keeps_the_quiet_queries(omega, oracle, pf):
+    # a query whose largest score comes first, next to queries (same wavefront) whose maximum rises
+    # in almost every later block of keys: the neighbours' rescaling must not touch it. Large scores
+    # (20 to 200), so that the exponent's reference has a rounding residual to get wrong.
+    rng = np.random.default_rng(77)
+    pos0, t, eps, ones = 4000, 1, 1e-6, np.ones(128, np.float32)
+    for m in (12, 516):  # the keys cut in chunks, and in one piece
+        c = omega.DecodeAttnCache(1, omega.round_max_pos(pos0 + m), 1e6)
+        c.set_norms(0, ones, ones)
+        keys, vals, heads = [], [], []
+        for h, level in enumerate((20.0, 60.0, 120.0, 200.0)):
+            u, v = np.linalg.qr(rng.standard_normal((128, 2)))[0].T
+            k = rng.standard_normal((pos0, 128))
+            k += level * v + 200.0 * np.arange(pos0)[:, None] / pos0 * u
+            k[0] += 3.0 * v
+            x = 0.1 * rng.standard_normal((pos0, 128)) + (np.arange(pos0) < pos0 / 2)[:, None]
+            k, x = oracle.f32_to_bf16(k.astype(np.float32)), oracle.f32_to_bf16(x.astype(np.float32))
+            c.write_rows(0, h, 0, k, x)
+            keys.append(oracle.bf16_to_f32(k).astype(np.float64))
+            vals.append(oracle.bf16_to_f32(x).astype(np.float64))
+            heads.append((level, u, v))
+        qkv = rng.standard_normal((m, 5120)).astype(np.float32)
+        for h, (level, u, v) in enumerate(heads):
+            qkv[t, 1024 * h:1024 * h + 1024] = np.tile(rot(v, -(pos0 + t)), 8)
+        quiet, loud = qkv.copy(), qkv.copy()
+        for n in (0, 2, 3):
+            for h, (level, u, v) in enumerate(heads):
+                loud[n, 1024 * h:1024 * h + 1024] = np.tile(rot(u, -(pos0 + n)), 8)
+                quiet[n, 1024 * h:1024 * h + 1024] = np.tile(rot(v, -(pos0 + n)), 8)
+        att = pf.PrefillAttention(c)
+        a = att.attend(0, pos0, m, loud, eps, 1.0)[0][t].reshape(4, 8, 128)
+        b = att.attend(0, pos0, m, quiet, eps, 1.0)[0][t].reshape(4, 8, 128)
+        np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
+        for h, (level, u, v) in enumerate(heads):
+            q = v / np.sqrt((v ** 2).mean() + eps)
+            rows = [c.read_row(0, h, pos0 + i) for i in (0, 1)]
+            k, x = (np.vstack([base] + [oracle.bf16_to_f32(r[i]).astype(np.float64)[None] for r in rows])
+                    for i, base in enumerate((keys[h], vals[h])))
+            w = np.exp((s := k @ q / np.sqrt(128)) - s.max())
+            want = (w / w.sum()) @ x
+            # q and the probabilities as bf16 pairs, 2^-17 each (a query's error in q moves all its scores
+            # along the shared direction alike and cancels), and a score of `level` summed in f32 over 16
+            # matrix-core products, 2^-24 of it each
+            assert rel_err(a[h], want[None]) <= 2 * 2.0 ** -17 + 16 * 2.0 ** -24 * level, (m, h)
+        c.free()
+
+
 def test_prefill_attention_refusals(omega, pf):
     c = omega.DecodeAttnCache(1, 256, 1e6)
     att = pf.PrefillAttention(c)
