@@ -30,6 +30,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <type_traits>
 #include <vector>
 
 #include "dattn.hpp"
@@ -781,6 +782,7 @@ __device__ __forceinline__ float pattn_factor(float m, float from, float to) {
 __global__ __launch_bounds__(512, 2) void k_pattn(const PattnArgs a) {
     __shared__ __align__(16) uint8_t kv[2][2][2][8192];  // [half][buffer][K | V]; also q rows, merge
     __shared__ float mls[2][4][64];
+    __shared__ float keep[8][16][64];                    // a wavefront's sums of 32 dims at a page edge
     const uint32_t tid = threadIdx.x, lane = lane_id();
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), qw = w & 3, kw = w >> 2;
     const uint32_t n = lane & 31, hl = lane >> 5;
@@ -827,6 +829,8 @@ __global__ __launch_bounds__(512, 2) void k_pattn(const PattnArgs a) {
     lds_sync();
     const uint32_t j = 4 * qw + (n >> 3), head = n & 7;          // the lane's query: token t0 + j
     const uint32_t pos = a.pos0 + t0 + min(j, valid - 1);
+    // the pages of the wavefront's first and last query
+    const uint32_t page0 = (a.pos0 + t0 + min(4 * qw, valid - 1)) >> 4, page1 = (a.pos0 + t0 + min(4 * qw + 3, valid - 1)) >> 4;
     bf16x8 qh[8], ql[8];                                         // dims 16 ks + 8 hl .. +8
     {
         float v[8][8];
@@ -880,7 +884,9 @@ __global__ __launch_bounds__(512, 2) void k_pattn(const PattnArgs a) {
         for (int i = 0; i < 16; ++i) O[dt][i] = 0.f;
     const uint32_t kt = (n & 0x13) | ((n & 4) << 1) | ((n & 8) >> 1);  // the key of K row n
     const uint32_t koff = kt * 256, kx = kt & 15;
-    auto compute = [&](int u, uint32_t b) {
+    // LAST: the blocks past the tile's first query, which hold keys that some query does not see
+    auto compute = [&](int u, uint32_t b, auto last) {
+        constexpr bool LAST = decltype(last)::value;
         const uint8_t *kb = kv[kw][u][0] + koff, *vb = kv[kw][u][1] + n * 32 + 16 * hl;
         f32x16 s;
 #pragma unroll
@@ -891,8 +897,7 @@ __global__ __launch_bounds__(512, 2) void k_pattn(const PattnArgs a) {
             s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k, qh[ks], s, 0, 0, 0);
             s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k, ql[ks], s, 0, 0, 0);
         }
-        if (kPattnBlock * b + kPattnBlock > a.pos0 + t0 + 1) {   // some query does not see some key
-            asm volatile("");                                    // stays a branch: most blocks skip it
+        if constexpr (LAST) {
 #pragma unroll
             for (int i = 0; i < 16; ++i)
                 if (kPattnBlock * b + 16 * (i >> 3) + 8 * hl + (i & 7) > pos) s[i] = -INFINITY;
@@ -912,6 +917,10 @@ __global__ __launch_bounds__(512, 2) void k_pattn(const PattnArgs a) {
             m_l = m_new;
             ref = to;
         }
+        // A key that a query does not see has probability 0, but 0 x a non-finite V is NaN, so a page goes
+        // only into the sums of the queries on it or past it: a wavefront with none of them skips it, one
+        // with some takes the others' sums back from LDS. (A branch in the loop over all blocks instead of
+        // a loop of its own for the last ones: 2048 tokens 104 us, copies in registers spilled, 112.)
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
             u32x4 hi, lo;
@@ -925,24 +934,46 @@ __global__ __launch_bounds__(512, 2) void k_pattn(const PattnArgs a) {
                 hi[e] = x;
                 lo[e] = y;
             }
+            const uint32_t page = 2 * b + kk;
+            if (LAST && page > page1) continue;
+            const bool edge = LAST && page > page0;
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) {
+                if (edge) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) keep[w][i][lane] = O[dt][i];
+                }
                 const bf16x8 v = as_bf16x8(*reinterpret_cast<const u32x4 *>(vb + 4096 * kk + 1024 * dt));
                 O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, as_bf16x8(hi), O[dt], 0, 0, 0);
                 O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, as_bf16x8(lo), O[dt], 0, 0, 0);
+                if (edge && page > pos >> 4) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) O[dt][i] = keep[w][i][lane];
+                }
             }
         }
     };
     const uint32_t steps = (b1 - b0 + 1) / 2;
+    const uint32_t whole = min(b1, (a.pos0 + t0 + 1) / kPattnBlock);  // the first of the last blocks
+    const uint32_t whole_steps = whole > b0 ? (whole - b0) / 2 : 0;
     stage(0);
     load(b0 + kw + 2);
     lds_sync();
-    for (uint32_t i = 0; i < steps; ++i) {
+    uint32_t i = 0;
+    for (; i < whole_steps; ++i) {
         const uint32_t b = b0 + kw + 2 * i;
         const int u = i & 1;
         stage(u ^ 1);
         load(b + 4);
-        if (b < b1) compute(u, b);  // uniform per wavefront
+        compute(u, b, std::false_type{});
+        lds_sync();
+    }
+    for (; i < steps; ++i) {
+        const uint32_t b = b0 + kw + 2 * i;
+        const int u = i & 1;
+        stage(u ^ 1);
+        load(b + 4);
+        if (b < b1) compute(u, b, std::true_type{});  // uniform per wavefront
         lds_sync();
     }
     // the two halves' states, lane by lane

@@ -449,6 +449,39 @@ def test_prefill_attention_rescale_keeps_the_quiet_queries(omega, oracle, pf):
         c.free()
 
 
+@pytest.mark.parametrize("pos0,m,bad", [
+    (5, 40, 18),        # the second page of a block, seen by a part of the tile's tokens
+    (5, 40, 34),        # the first page of the block after
+    (5, 40, 44),        # the last token
+    (614, 70, 625),     # the page boundary (624) inside a group of four tokens
+    (3001, 30, 3025),   # the keys cut in chunks
+    (2001, 600, 2018),
+])
+def test_prefill_attention_keeps_a_bad_value_in_its_page(omega, pf, pos0, m, bad):
+    # the V row of position `bad` is an infinity and a NaN: only tokens on its page or after it may
+    # see them, the rows of the pages before are those of a finite V bit for bit
+    rng = np.random.default_rng(pos0 + m)
+    c = omega.DecodeAttnCache(1, omega.round_max_pos(pos0 + m), 1e6)
+    c.set_norms(0, np.ones(128, np.float32), np.ones(128, np.float32))
+    for h in range(4):
+        kv = (rng.standard_normal((2, pos0, 128)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+        c.write_rows(0, h, 0, kv[0], kv[1])
+    qkv = rng.standard_normal((m, 5120)).astype(np.float32)
+    att = pf.PrefillAttention(c)
+    clean = att.attend(0, pos0, m, qkv, 1e-6, 1.0)[0]
+    qkv[bad - pos0, 4608:4608 + 512:128] = np.inf
+    qkv[bad - pos0, 4609:4609 + 512:128] = np.nan
+    got = att.attend(0, pos0, m, qkv, 1e-6, 1.0)[0]
+    before = bad // 16 * 16 - pos0
+    assert before > 0
+    np.testing.assert_array_equal(got[:before].view(np.uint32), clean[:before].view(np.uint32))
+    seen = got[bad - pos0:].reshape(-1, 32, 128)
+    assert not np.isfinite(seen[:, :, :2]).any()
+    np.testing.assert_array_equal(got.reshape(m, 32, 128)[:, :, 2:].view(np.uint32),
+                                  clean.reshape(m, 32, 128)[:, :, 2:].view(np.uint32))
+    c.free()
+
+
 def test_prefill_attention_refusals(omega, pf):
     c = omega.DecodeAttnCache(1, 256, 1e6)
     att = pf.PrefillAttention(c)
