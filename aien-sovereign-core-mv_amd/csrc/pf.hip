@@ -146,6 +146,7 @@ __global__ __launch_bounds__(256) void k_pf_quant(const PfQuantArgs a) {
 struct PfGemmArgs {
     uint32_t n = 0, k = 0, layout = 0, ntiles = 0;
     uint32_t by_cols = 0;  // an XCD takes a range of column spans (else a range of tiles)
+    uint32_t per = 0;      // workgroups of an XCD's range
     const PfTile *tiles = nullptr;
     const uint32_t *rowidx = nullptr;  // nullptr: output row r reads activation row r
     const uint8_t *xq = nullptr;       // [rows][k] e4m3
@@ -298,17 +299,19 @@ __device__ __forceinline__ void pf_qgemm_wg(const PfGemmArgs &a, Lds &L, uint64_
     }
 }
 
-// Grid: 8 x ceil(column spans x tiles / 8) workgroups; workgroup b runs on XCD b % 8, and each XCD
-// takes one contiguous range of the (tile, span) list, ordered so that what its workgroups share
-// stays in its L2: by tile, an expert's weights and a tile's activation rows are read into one L2
-// only; by span, a span's weights.
+// Grid: at least 8 x ceil(column spans x tiles / 8) workgroups, in rows of at most kPfGridX (a multiple
+// of 8; the threads of a grid's row must stay below 2^32); workgroup b of all of them runs on XCD
+// b % 8, and each XCD takes one contiguous range of the (tile, span) list, ordered so that what its
+// workgroups share stays in its L2: by tile, an expert's weights and a tile's activation rows are read
+// into one L2 only; by span, a span's weights.
+constexpr uint32_t kPfGridX = 1u << 20;
+
 template <int LAYOUT, bool PAIR>
 __global__ __launch_bounds__(PAIR ? 512 : 256, PAIR ? 2 : 3) void k_pf_qgemm(const PfGemmArgs a) {
     constexpr int RW = PAIR ? 4 : 2;
     __shared__ __align__(16) PfLds<64 * RW, PAIR ? 128 : 64> L;
     const uint32_t nx = a.n / (64 * RW);
-    const uint32_t total = nx * a.ntiles, per = gridDim.x >> 3;
-    const uint32_t id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    const uint32_t total = nx * a.ntiles, wg = blockIdx.y * kPfGridX + blockIdx.x, id = (wg & 7) * a.per + (wg >> 3);
     if (id >= total) return;
     const uint32_t x = a.by_cols ? id / a.ntiles : id % nx, t = a.by_cols ? id % a.ntiles : id / nx;
     const cu32 *tw = as_const_u32(a.tiles + t);
@@ -996,9 +999,11 @@ int omega_gpu_pf_qgemm(uint32_t n, uint32_t k, uint32_t layout, uint64_t tiles_v
     // of 3000 tokens 157 against 170). gate|up gains nothing (2000 tokens 172 against 151 us).
     const bool pair = layout == kPfLayoutPlain && !a.by_cols && n % 256 == 0 &&
                       (uint64_t)(n / 256) * ntiles * (k / 128) >= 10240;
-    const uint64_t wgs = ((uint64_t)(n / (pair ? 256 : 128)) * ntiles + 7) / 8 * 8;
+    const uint32_t wgs = (n / (pair ? 256 : 128) * ntiles + 7) / 8 * 8;  // at most 1022 x 65535
+    const uint32_t gx = std::min(wgs, kPfGridX), gy = (wgs + gx - 1) / gx;
+    a.per = gx * gy / 8;
     return pf_timed(F_SESSION, 1, ns, [&](hipStream_t st) {
-        const dim3 grid((uint32_t)wgs), block(pair ? 512 : 256);
+        const dim3 grid(gx, gy), block(pair ? 512 : 256);
         if (layout == kPfLayoutSwiglu) OMEGA_LAUNCH((k_pf_qgemm<kPfLayoutSwiglu, false>), grid, block, 0, st, a);
         else if (pair) OMEGA_LAUNCH((k_pf_qgemm<kPfLayoutPlain, true>), grid, block, 0, st, a);
         else OMEGA_LAUNCH((k_pf_qgemm<kPfLayoutPlain, false>), grid, block, 0, st, a);

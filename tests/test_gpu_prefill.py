@@ -233,6 +233,33 @@ def test_qgemm_tile_runs(omega, oracle, pf, n, k, counts):
     T.free()
 
 
+def test_qgemm_more_workgroups_than_one_grid_dimension_holds(omega, oracle, pf):
+    # 1022 column spans x 16500 tiles of 256 threads are more than 2^32 threads; three tiles have rows,
+    # the others none
+    rng = np.random.default_rng(31)
+    n, k, ntiles, rows = 130816, 128, 16500, {0: (0, 3), 8250: (3, 64), 16499: (67, 1)}
+    assert n // 128 * ntiles * 256 >= 1 << 32
+    w, s = oracle.synth_fp8(14, 6, 1, n, k)
+    wd, sd = dev_from(omega, w), dev_from(omega, oracle.bf16_to_f32(s).astype(np.float32))
+    q, qs = run_quant(omega, pf, rng.standard_normal((68 + pf.qgemm_bm(), k)).astype(np.float32), pf.IN_F32)
+    xq, xs = dev_from(omega, q), dev_from(omega, qs)
+    tiles = np.zeros(ntiles, pf.TILE_DTYPE)
+    tiles["w_va"], tiles["s_va"] = wd.ptr.value, sd.ptr.value
+    for t, (row0, cnt) in rows.items():
+        tiles["row0"][t], tiles["cnt"][t] = row0, cnt
+    td = dev_from(omega, tiles.view(np.uint8))
+    yd = dev_from(omega, np.full(69 * (n // 2), 0x4040, np.uint16))
+    pf.qgemm(n, k, pf.SWIGLU_NAT, td.ptr, ntiles, 0, xq.ptr, xs.ptr, yd.ptr)
+    y = yd.download(np.uint16, 69 * (n // 2)).reshape(69, n // 2)
+    assert (y[68] == 0x4040).all()
+    X, W = dequant_rows(oracle, q, qs), dequant_weights(oracle, w, s)[0]
+    for r in (0, 2, 3, 40, 66, 67):
+        gu = W @ X[r]
+        want = gu[:n // 2] / (1 + np.exp(-gu[:n // 2])) * gu[n // 2:]
+        got = oracle.bf16_to_f32(y[r])
+        assert np.all(np.abs(got - want) <= np.abs(want) * 2.0 ** -8 + GEMM_TOL * np.abs(want).max()), r
+
+
 def sequential_logits(wq_rows, x):
     """logits[r][ex] = the f32 sum from -0.0, in column order, of f32-rounded products, every
     row and expert at once (numpy float32 arithmetic rounds each product and each sum)"""
