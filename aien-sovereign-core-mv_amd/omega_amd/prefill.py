@@ -330,7 +330,7 @@ class WholePromptPrefill:
                  qkv=PfMem(m * qkv_n * 4), att=PfMem(m * qd * 4), oproj=PfMem(m * h * 4),
                  logits=PfMem(mt * e * 4), act=PfMem(g * i * 2), aq=PfMem((g + bm) * i),
                  a_s=PfMem((g + bm) * (i // BLOCK) * 4), down=PfMem(g * h * 4), moe=PfMem(m * h * 4),
-                 plan=PfMem(at[-1]), dense=PfMem(dense_tiles * TILE_BYTES))
+                 plan=PfMem(at[-1]), dense=PfMem(max(1, dense_tiles) * TILE_BYTES))
         self.bufs = b
         return b
 
@@ -357,6 +357,8 @@ class WholePromptPrefill:
     def _put_dense(self, b, m):
         """the tile tables of m rows over every layer's q|k|v and o weights, [layer][q|k|v, o][tile]"""
         nt = -(-m // self.bm)
+        if not self.layers:  # a model of its embedding and final norm alone
+            return nt
         tab = np.zeros((len(self.layers), 2, nt), TILE_DTYPE)
         for j, name in enumerate(("qkv", "o")):
             tab["w_va"][:, j] = np.array([L["ent"][name][0] for L in self.layers])

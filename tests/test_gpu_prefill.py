@@ -613,6 +613,18 @@ def test_whole_prompt_matches_the_w8a8_oracle(omega, oracle, pf, small):
     print(f"whole-prompt stages within bars, routing flips {flips}")
 
 
+@pytest.mark.parametrize("m", [1, 130])
+def test_whole_prompt_without_layers(omega, oracle, pf, m):
+    rng = np.random.default_rng(12)
+    emb, norm = rng.standard_normal((7, 2048)).astype(np.float32), (1 + 0.1 * rng.standard_normal(2048)).astype(np.float32)
+    cache = omega.DecodeAttnCache(1, 256, 1e6)
+    wp = pf.WholePromptPrefill([], norm, lambda t: emb[t], cache, 1e-6)
+    tokens = rng.integers(0, 7, m).tolist()
+    np.testing.assert_array_equal(wp.run(tokens, 0), oracle.rmsnorm(emb[tokens[-1]], norm, 1e-6))
+    wp.free()
+    cache.free()
+
+
 def rmsnorm_last(oracle, m, x):
     return oracle.rmsnorm(x[-1], m.final_norm(), m.cfg.eps)
 
