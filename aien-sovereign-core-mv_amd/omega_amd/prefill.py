@@ -311,19 +311,11 @@ class WholePromptPrefill:
         g = m * top_k
         kmax = max(h, qd)
         mt = -(-m // self.t) * self.t
-        max_tiles = -(-g // bm) + e
-        # the layer's plan, written by the host next to the logits it is made from and moved by one
-        # copy (byte offsets): activation row of each grouped row, grouped row and weight of each
-        # (token, slot), the tile tables of gate|up and down
-        up16 = lambda v: (v + 15) // 16 * 16
-        at = [0]
-        for nb in ((g + bm) * 4, g * 4, g * 4, max_tiles * TILE_BYTES, max_tiles * TILE_BYTES):
-            at.append(at[-1] + up16(nb))
-        base = up16(mt * e * 4)
+        base, at = self._plan_at(m)
         dense_tiles = len(self.layers) * 2 * -(-m // bm)
         # HOST buffers are the CPU's side (written or read in place); the kernels read and write
         # DEVICE buffers, and the copies between them are DMA (omega_gpu_pf_copy_va)
-        b = dict(m=m, max_tiles=max_tiles, plan_at=at, plan_stage=base,
+        b = dict(m=m,
                  stage=PfMem(max(max(mt * max(h, e), m * qkv_n, g * h) * 4 + g * 8, base + at[-1],
                                  dense_tiles * TILE_BYTES), host=True),
                  x=PfMem(m * h * 4), xin=PfMem(mt * h * 4), xq=PfMem((m + bm) * kmax), xs=PfMem((m + bm) * (kmax // BLOCK) * 4),
@@ -333,6 +325,21 @@ class WholePromptPrefill:
                  plan=PfMem(at[-1]), dense=PfMem(max(1, dense_tiles) * TILE_BYTES))
         self.bufs = b
         return b
+
+    def _max_tiles(self, m):
+        return -(-m * self.top_k // self.bm) + self.e
+
+    def _plan_at(self, m):
+        """A layer's plan for m tokens, written by the host next to the logits it is made from and moved
+        by one copy: its place in the staging buffer, past the logits, and the byte offsets in it and in
+        the device's plan buffer of the activation row of each grouped row, the grouped row and the
+        weight of each (token, slot), the tile tables of gate|up and down, and its end."""
+        up16 = lambda v: (v + 15) // 16 * 16
+        g, tab = m * self.top_k, self._max_tiles(m) * TILE_BYTES
+        at = [0]
+        for nb in ((g + self.bm) * 4, g * 4, g * 4, tab, tab):
+            at.append(at[-1] + up16(nb))
+        return up16(-(-m // self.t) * self.t * self.e * 4), at
 
     def _up(self, dst, arr):
         """host rows -> a device buffer through the staging buffer"""
@@ -370,26 +377,26 @@ class WholePromptPrefill:
 
     def _put_plan(self, b, m, ent):
         """Routes the m token rows of the staged logits (omega_gpu_pf_moe_plan) and moves the layer's
-        plan to the device. Returns the plan (views of the staging buffer: ids, weights, a2g) and its
-        tile count."""
-        e, top_k, at = self.e, self.top_k, b["plan_at"]
+        plan to the device. Returns the plan (views of the staging buffer: ids, weights, a2g), its
+        tile count and the device addresses of its parts."""
+        e, top_k, g = self.e, self.top_k, m * self.top_k
+        base, at = self._plan_at(m)
         stage = b["stage"].host(np.uint8)
-        addr = [b["stage"].mem.cpu + b["plan_stage"] + v for v in at]
+        addr = [b["stage"].mem.cpu + base + v for v in at]
         ids, counts = np.empty((m, top_k), np.uint32), np.empty(e, np.uint32)
         _pf_check(lib().omega_gpu_pf_moe_plan(m, e, top_k, b["stage"].mem.cpu, ids.ctypes.data, addr[2],
                                               counts.ctypes.data, addr[0], addr[1], None), "pf moe plan")
         n = 0
         for off, (w, sc) in ((3, ent["gu"]), (4, ent["dn"])):
             n = lib().omega_gpu_pf_qgemm_tiles_va(e, w.ctypes.data, sc.ctypes.data, counts.ctypes.data, addr[off],
-                                                  b["max_tiles"])
+                                                  self._max_tiles(m))
             if n == 0:
-                raise OmegaGpuError(-1, f"tile table larger than its region of {b['max_tiles']} entries")
+                raise OmegaGpuError(-1, f"tile table larger than its region of {self._max_tiles(m)} entries")
         # row indices past the last row are read with a tile of bm rows and must name a row
-        g = m * top_k
-        stage[b["plan_stage"] + 4 * g:b["plan_stage"] + 4 * (g + self.bm)] = 0
-        copy_va(b["plan"].va, b["stage"].va + b["plan_stage"], at[-1])
-        view = lambda i, dt: stage[b["plan_stage"] + at[i]:b["plan_stage"] + at[i] + 4 * g].view(dt)
-        return ids, view(2, np.float32).reshape(m, top_k), view(1, np.uint32), n
+        stage[base + 4 * g:base + 4 * (g + self.bm)] = 0
+        copy_va(b["plan"].va, b["stage"].va + base, at[-1])
+        view = lambda i, dt: stage[base + at[i]:base + at[i] + 4 * g].view(dt)
+        return ids, view(2, np.float32).reshape(m, top_k), view(1, np.uint32), n, [b["plan"].va + v for v in at]
 
     def run(self, tokens, pos0, trace=None):
         """Tokens at positions pos0 .. pos0 + m - 1 through every layer; returns the last token's
@@ -429,8 +436,7 @@ class WholePromptPrefill:
             logits = self._down(b["logits"], np.float32, m * e)
             if trace is not None:
                 trace.setdefault("logits", []).append(logits.reshape(m, e).copy())
-            ids, wts, a2g, nt = self._put_plan(b, m, ent)
-            plan = [b["plan"].va + v for v in b["plan_at"]]
+            ids, wts, a2g, nt, plan = self._put_plan(b, m, ent)
             if trace is not None:
                 trace.setdefault("wts", []).append(wts.copy())
                 trace.setdefault("a2g", []).append(a2g.copy())

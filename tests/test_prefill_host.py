@@ -122,6 +122,67 @@ def test_routing_plan_in_a_forked_child(pf):
         np.testing.assert_array_equal(a, b)
 
 
+def test_the_drivers_plan_copy_follows_the_prompt(pf, monkeypatch):
+    """What a layer's plan copy moves depends on the prompt at hand, not on the longest before it, and
+    what arrives is that prompt's plan (the driver's buffers and copies stand in host memory here)."""
+    class Mem:
+        def __init__(self, nbytes, host=False):
+            self.buf = np.zeros((nbytes + 15) // 16 * 16 + 16, np.uint8)
+            self.va = (self.buf.ctypes.data + 15) // 16 * 16
+            self.nbytes, self.mem = nbytes, self
+
+        cpu = property(lambda self: self.va)
+
+        def free(self):
+            pass
+
+        def host(self, dtype=np.uint8):
+            at = self.va - self.buf.ctypes.data
+            return self.buf[at:at + self.nbytes].view(dtype)
+
+    moved = []
+
+    def copy_va(dst, src, nbytes):
+        moved.append(nbytes)
+        C.memmove(dst, src, nbytes)
+
+    monkeypatch.setattr(pf, "PfMem", Mem)
+    monkeypatch.setattr(pf, "copy_va", copy_va)
+
+    class Cache:
+        pass
+
+    class Tensor:
+        def entry(self, x):
+            return 4096 * (x + 1), 16 * (x + 1)
+
+    t, e, top = Tensor(), 128, 8
+    layer = dict(qkv=t, o=t, gate_up=t, down=t, input_norm=np.ones(2048), post_norm=np.ones(2048),
+                 router=np.zeros((e, 2048), np.float32))
+    rng = np.random.default_rng(13)
+
+    def plan(wp, m):
+        b = wp._ensure(m)
+        lg = rng.standard_normal((m, e)).astype(np.float32)
+        b["stage"].host(np.float32)[:m * e] = lg.reshape(-1)
+        moved.clear()
+        ids, wts, a2g, nt = wp._put_plan(b, m, wp.layers[0]["ent"])[:4]
+        assert len(moved) == 1
+        ref_ids, ref_wts, counts, gtok, ref_a2g = pf.moe_plan(lg, m, e, top)
+        np.testing.assert_array_equal(ids, ref_ids)
+        dev = b["plan"].host(np.uint8)
+        np.testing.assert_array_equal(dev[:4 * m * top].view(np.uint32), gtok)
+        for want in (ref_a2g, ref_wts, pf.build_tiles(wp.bm, *wp.layers[0]["ent"]["gu"], counts)):
+            assert want.tobytes() in dev[:moved[0]].tobytes()
+        return moved[0]
+
+    wp = pf.WholePromptPrefill([layer], np.ones(2048, np.float32), None, Cache(), 1e-6)
+    short = plan(wp, 64)
+    assert short <= 3 * 4 * 64 * top + 4 * wp.bm + 2 * pf.TILE_BYTES * (e + 64 * top // wp.bm) + 5 * 16
+    assert plan(wp, 2000) > short
+    assert plan(wp, 64) == short and plan(wp, 1999) > short
+
+
 def test_host_rmsnorm_matches_the_oracle(pf, oracle):
     rng = np.random.default_rng(4)
     x = (rng.standard_normal((5, 2048)) * 3).astype(np.float32)
