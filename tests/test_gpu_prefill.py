@@ -201,17 +201,19 @@ def test_qgemm_grouped_swiglu_and_down(omega, oracle, pf):
     DN.free()
 
 
-@pytest.mark.parametrize("n,k,counts", [
-    (128, 128, [1]),                                   # one k-block, one row
-    (384, 384, [64, 1, 63]),                           # odd k-blocks, tiles at and beside 64 rows
-    (256, 256, [17, 0, 65, 128]),
-    (256, 640, [31, 32, 33, 96, 97]),                  # tiles at and beside 32 rows, the short tiles' form
-    # the paired form (256-row workgroups over two tiles of a run): runs of 1 to 5 tiles, full and
+@pytest.mark.parametrize("n,k,counts,paired", [
+    (128, 128, [1], False),                            # one k-block, one row
+    (384, 384, [64, 1, 63], False),                    # odd k-blocks, tiles at and beside 64 rows
+    (256, 256, [17, 0, 65, 128], False),
+    (256, 640, [31, 32, 33, 96, 97], False),           # tiles at and beside 32 rows, the short tiles' form
+    # the paired form (256-row workgroups over two tiles of a run): runs of 1 to 10 tiles, full and
     # partial ends, so pairs start at even and at odd tiles of the table
-    (512, 12288, [64, 128, 65, 1, 192, 320, 129, 63, 256, 200, 64, 300, 130, 640, 511]),
-    (256, 3968, [4096 + 3, 8192]),                     # long runs, an odd number of k-blocks
+    (512, 12288, [64, 128, 65, 1, 192, 320, 129, 63, 256, 200, 64, 300, 130, 640, 511], False),
+    (512, 12288, [64, 128, 65, 1, 192, 320, 129, 63, 256, 200, 64, 300, 130, 640, 511, 192, 31], True),
+    (256, 3968, [4096 + 3, 8192], False),              # long runs, an odd number of k-blocks
+    (512, 3968, [4096 + 3, 8192], True),               # the same in pairs: more than 64 tiles to look back
 ])
-def test_qgemm_tile_runs(omega, oracle, pf, n, k, counts):
+def test_qgemm_tile_runs(omega, oracle, pf, n, k, counts, paired):
     rng = np.random.default_rng(n + k)
     E, g, bm = len(counts), sum(counts), pf.qgemm_bm()
     w, s = oracle.synth_fp8(13, 5, E, n, k)
@@ -219,6 +221,8 @@ def test_qgemm_tile_runs(omega, oracle, pf, n, k, counts):
     q, qs = run_quant(omega, pf, rng.standard_normal((g + bm, k)).astype(np.float32), pf.IN_F32)
     xq, xs = dev_from(omega, q), dev_from(omega, qs)
     tiles = pf.build_tiles(bm, [T.entry(e)[0] for e in range(E)], [T.entry(e)[1] for e in range(E)], counts)
+    # the rule of omega_gpu_pf_qgemm for the paired form: its cases must stay on its side of it
+    assert paired == (n % 256 == 0 and 64 * len(tiles) >= n and n // 256 * len(tiles) * (k // 128) >= 10240)
     td = dev_from(omega, tiles.view(np.uint8))
     yd = dev_from(omega, np.full((g + 1) * n, 7.0, np.float32))
     pf.qgemm(n, k, pf.PLAIN, td.ptr, len(tiles), 0, xq.ptr, xs.ptr, yd.ptr)
@@ -338,8 +342,8 @@ def test_residual_norm_row_edges(omega, pf, k, rows, off):
 
 @pytest.mark.parametrize("N,first", [(300, 100), (1300, 1030)])
 def test_prefill_attention_equals_the_decode_attention(omega, oracle, pf, N, first):
-    # (1300, 1030): contexts past 1024 take the 4-token query tiles, the first call spans two
-    # sub-batches of 1024 + 6 tokens (a partial tile) and the second starts at an unaligned 1030
+    # (1300, 1030): the first call takes its keys in one piece and ends in a partial tile, the second
+    # starts at an unaligned 1030 and cuts them in chunks
     rng = np.random.default_rng(8)
     layers, eps = 2, 1e-6
     qn = (1 + 0.1 * rng.standard_normal((layers, 128))).astype(np.float32)
@@ -357,7 +361,7 @@ def test_prefill_attention_equals_the_decode_attention(omega, oracle, pf, N, fir
     dec = np.stack([a.attend(layer, p, qkv[p], eps)[0] for p in range(N)])
     att = pf.PrefillAttention(b)
     o1, info = att.attend(layer, 0, first, qkv[:first], eps, 1.0)
-    # work items: (query tile of consecutive tokens, chunk of 32 pages) pairs, one wavefront per kv head
+    # work items: (tile of 16 query tokens, chunk of the keys) pairs, one workgroup per kv head
     assert info.m == first and 1 <= info.chunks <= 4 * first and info.grid_x == 4 * info.chunks
     o2, _ = att.attend(layer, first, N - first, qkv[first:], eps, 1.0)
     pre = np.vstack([o1, o2])
@@ -509,6 +513,57 @@ def test_prefill_attention_keeps_a_bad_value_in_its_page(omega, pf, pos0, m, bad
     c.free()
 
 
+def test_prefill_attention_of_two_sub_batches(omega, pf):
+    # more than 4096 tokens, against the decode attention of every token on another cache: the second
+    # sub-batch (37 tokens from an unaligned position) has its own rows, position and chunk count (9
+    # chunks of up to 4138 keys), the first takes its keys in one piece
+    rng = np.random.default_rng(14)
+    pos0, m = 5, 4096 + 37
+    a, b = (omega.DecodeAttnCache(1, omega.round_max_pos(pos0 + m), 1e6) for _ in range(2))
+    qkv = rng.standard_normal((pos0 + m, 5120)).astype(np.float32)
+    for c in (a, b):
+        c.set_norms(0, np.ones(128, np.float32), np.ones(128, np.float32))
+    want = [a.attend(0, p, qkv[p], 1e-6)[0] for p in range(pos0 + m)]
+    for p in range(pos0):
+        b.attend(0, p, qkv[p], 1e-6)
+    got, info = pf.PrefillAttention(b).attend(0, pos0, m, qkv[pos0:], 1e-6, 1.0)
+    assert info.splits == 9 and info.chunks == 4096 // 16 + 3 * 9
+    for t in (0, 1, 10, 11, 2047, 4079, 4080, 4094, 4095, 4096, 4097, 4111, 4112, 4128, m - 1):
+        # q and the probabilities as bf16 pairs (2^-17 each) on scores of up to about 12, on both sides
+        assert rel_err(got[t], want[pos0 + t]) <= 5e-4, t
+    for h in range(4):
+        for p in (0, pos0 + 4095, pos0 + 4096, pos0 + m - 1):
+            for x, y in zip(a.read_row(0, h, p), b.read_row(0, h, p)):
+                np.testing.assert_array_equal(x, y)
+    a.free()
+    b.free()
+
+
+@pytest.mark.parametrize("n,split,same", [
+    (1200, 601, True),    # both calls of the split take the keys in one piece, as the whole call does
+    (700, 601, False),    # the second call cuts its keys in chunks
+])
+def test_prefill_attention_rows_of_a_split_call(omega, pf, n, split, same):
+    # a split that is no multiple of the 4 tokens of a wavefront or the 16 of a tile, over many blocks
+    # of keys: a row's arithmetic depends on the call only through the chunks of the keys
+    rng = np.random.default_rng(n)
+    c = omega.DecodeAttnCache(1, omega.round_max_pos(n), 1e6)
+    c.set_norms(0, np.ones(128, np.float32), np.ones(128, np.float32))
+    qkv = rng.standard_normal((n, 5120)).astype(np.float32)
+    att = pf.PrefillAttention(c)
+    want, info = att.attend(0, 0, n, qkv, 1e-6, 1.0)
+    one, i1 = att.attend(0, 0, split, qkv[:split], 1e-6, 1.0)
+    two, i2 = att.attend(0, split, n - split, qkv[split:], 1e-6, 1.0)
+    assert info.splits == i1.splits == 1 and (i2.splits == 1) == same
+    np.testing.assert_array_equal(one, want[:split])
+    if same:
+        np.testing.assert_array_equal(two, want[split:])
+    else:  # the chunks' references round the probabilities' bf16 pairs otherwise: 2^-17 on either side
+        for t in range(split, n):
+            assert rel_err(two[t - split], want[t]) <= 2 * 2.0 ** -17, t
+    c.free()
+
+
 def test_prefill_attention_refusals(omega, pf):
     c = omega.DecodeAttnCache(1, 256, 1e6)
     att = pf.PrefillAttention(c)
@@ -630,9 +685,9 @@ def rmsnorm_last(oracle, m, x):
 
 
 def test_whole_prompt_is_row_independent(omega, oracle, pf, small):
-    # a prompt in two calls (the second at pos0 = 24) gives the one-call results bit for bit: no
-    # row's arithmetic depends on the other rows of a launch, and the cache it leaves holds the
-    # same K / V rows
+    # a prompt in two calls (the second at pos0 = 24) gives the one-call results bit for bit: a row's
+    # arithmetic depends on its call only through the chunks of the attention's keys, here one in
+    # every call, and the cache it leaves holds the same K / V rows
     m, wp, cache = small
     rng = np.random.default_rng(10)
     tokens = rng.integers(0, 4096, 48).tolist()
