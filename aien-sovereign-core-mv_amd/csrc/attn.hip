@@ -772,10 +772,10 @@ __device__ __forceinline__ float pattn_factor(float m, float from, float to) {
 //
 // Bounded by the matrix cores and the work per score on the VALU (32 products of 32 cycles and about
 // 150 VALU operations per wavefront and step; the clock drops to 1.9 GHz), not by K / V bytes: 128
-// queries share a block's 16 KiB. At 2500 tokens behind 5000 it runs 0.86 PFLOP/s of bf16 products,
+// queries share a block's 16 KiB. At 2500 tokens behind 5000 it runs 1.0 PFLOP/s of bf16 products,
 // where a plain 8192^3 bf16 product reaches 1.2 on this card. Measured (append, attention and
-// combine; wavefronts of up to 4 tokens that read their pages themselves before): 2048 tokens 402
-// -> 98 us, 512 tokens 69 -> 30, 333 tokens behind 3700 202 -> 68, 16 behind 6000 75 -> 35. 64
+// combine; wavefronts of up to 4 tokens that read their pages themselves before): 2048 tokens 381
+// -> 98 us, 512 tokens 67 -> 30, 333 tokens behind 3700 181 -> 65, 16 behind 6000 72 -> 33. 64
 // queries a wavefront (4 wavefronts, the q operands in AGPRs) took 149 us at 2048 tokens, four
 // wavefronts a workgroup and two workgroups a CU 108; operands read ahead of their products,
 // wavefront priorities and two score accumulators changed nothing.

@@ -3,9 +3,9 @@
 Mirrors crates/aien-omega-pf (the safe wrappers: PfMem, OmegaPfDevice, OmegaPrefillAttention,
 build_tiles, pack_router) and the driver WholePromptPrefill (crates/aien-inference-abi/src/
 qwen3_moe_omega_prefill.rs:483-760) in its device-host form (qwen3_moe_omega_prefill/devhost.rs:
-router logits and the MoE combine on the chip). The host steps stay on the host as in the
-reference: the RMSNorms (f64 sum of squares), the residual adds, the routing plan
-(MoeBatchPlan::from_logits, moe_plan.rs:86-171) and the expert sort.
+router logits and the MoE combine on the chip). The residual adds and RMSNorms run on the chip too
+(omega_gpu_pf_residual_norm); the routing plan (MoeBatchPlan::from_logits, moe_plan.rs:86-171) and
+the expert sort stay on the host as in the reference.
 
 The whole prompt goes through every layer with a fixed launch count per layer: quantise x, the
 q|k|v GEMM, the prefill attention, quantise the attention rows, the o GEMM, the router logits,
@@ -392,7 +392,8 @@ class WholePromptPrefill:
                                                   self._max_tiles(m))
             if n == 0:
                 raise OmegaGpuError(-1, f"tile table larger than its region of {self._max_tiles(m)} entries")
-        # row indices past the last row are read with a tile of bm rows and must name a row
+        # the boundary lets a GEMM read row indices up to a whole tile past a tile's first row (the
+        # library's own reads the tile's rows only): they name a row
         stage[base + 4 * g:base + 4 * (g + self.bm)] = 0
         copy_va(b["plan"].va, b["stage"].va + base, at[-1])
         view = lambda i, dt: stage[base + at[i]:base + at[i] + 4 * g].view(dt)

@@ -505,8 +505,8 @@ typedef struct OmegaGpuPfTile {
     uint32_t row0, cnt;
     uint64_t pad;
 } OmegaGpuPfTile;
-/* lib.rs:362-376. Here chunks counts the call's work items, (tile of consecutive query tokens: 4
- * from a context of 1024 on, else 1; chunk of 32 pages) pairs, and grid_x = 4 kv heads x chunks */
+/* lib.rs:362-376. Here chunks counts the call's work items, (tile of 16 consecutive query tokens,
+ * chunk of the keys) pairs, grid_x = 4 kv heads x chunks, and splits is the most chunks of a tile */
 typedef struct OmegaGpuPrefillAttnInfo {
     uint32_t layer, pos0, m, chunks, grid_x, grid_y, threads, splits, per_split;
     uint64_t elapsed_ns, call_ns;
@@ -529,8 +529,8 @@ uint32_t omega_gpu_pf_qgemm_bm(void);                                           
 uint32_t omega_gpu_pf_qgemm_tiles_va(uint32_t experts, const uint64_t *w_va, const uint64_t *s_va,
                                      const uint32_t *counts, void *tab, uint32_t max);
 /* :411-424: for every tile, output rows row0 .. row0 + cnt of W_expert x dequant(activation row
- * rowidx[row] (or row when rowidx_va is 0)); the kernel reads activation rows (and row indices)
- * up to row0 + bm - 1 of every tile */
+ * rowidx[row] (or row when rowidx_va is 0)); the boundary lets the kernel read activation rows and
+ * row indices up to row0 + bm - 1 of every tile (this one reads the tile's own cnt rows) */
 int omega_gpu_pf_qgemm(uint32_t n, uint32_t k, uint32_t layout, uint64_t tiles_va, uint32_t ntiles,
                        uint64_t rowidx_va, uint64_t xq_va, uint64_t xs_va, uint64_t y_va, uint64_t *ns);
 uint32_t omega_gpu_pf_router_rows(void);                                               /* :430 */
