@@ -687,8 +687,8 @@ struct PattnArgs {
     const float *rope_cos = nullptr, *rope_sin = nullptr;
     float eps = 1e-6f;
     uint32_t nch = 1;            // chunks of the keys per tile
-    float *part = nullptr;       // nch > 1: [m][nch][32][kPartStride]
-    float *out = nullptr;        // nch 1: [m][32][128]
+    float *part = nullptr;       // [m][nch][32][kPartStride]
+    float *out = nullptr;        // [m][32][128]: nch 1 and the rows written directly, else partials
     float out_scale = 1.0f;
 };
 
@@ -1003,7 +1003,7 @@ __global__ __launch_bounds__(512, 2) void k_pattn(const PattnArgs a) {
     if (j >= valid) return;
     float *dst;
     float f = 1.f;
-    if (a.nch == 1) {
+    if (a.out) {
         dst = a.out + (size_t)(t0 + j) * 4096 + (h * 8 + head) * 128;
         f = a.out_scale / l_l;
     } else {
@@ -2055,6 +2055,10 @@ int omega_gpu_decode_attn_cache_import_dev(OmegaGpuDecodeAttnCache *c, uint32_t 
 // Sub-batches of at most kPattnSub tokens (a multiple of the query tile): a launch's K / V append
 // goes before its attention, and a sub-batch sees the ones before it in the cache.
 constexpr uint32_t kPattnSub = 4096;
+// Where the output rows lie over the q|k|v rows, a workgroup must not write its rows while others read
+// theirs: every tile goes through partials, whose combine writes, in sub-batches whose partials fit
+// the scratch (rows written over the q|k|v rows themselves stay behind the sub-batches still to come).
+constexpr uint32_t kPattnSubOver = 1024;
 
 // Chunks of the keys for a call of m tokens from pos0: with fewer workgroups than CUs the keys are
 // cut, into pieces of at least 512 keys (16 blocks), until the workgroups fill the chip. A tile
@@ -2069,8 +2073,8 @@ static uint32_t pattn_chunks(uint32_t pos0, uint32_t m) {
 // The scratch that a prefill attention call of m tokens from pos0 asks for. The serving reservation
 // and its seal are written against this size (a sealed library refuses a call that asks for more
 // than it holds), so it stays what it was when a call held 1024 prepared query rows, their plan and
-// a partial per token and 512 keys. The partials of this form (at most 512 tokens in at most that
-// many chunks) fit in it.
+// a partial per token and 512 keys. The partials of this form (at most 512 tokens, or kPattnSubOver, in
+// at most that many chunks) fit in it.
 static size_t pattn_scratch(uint32_t pos0, uint32_t m) {
     const size_t sub = std::min(1024u, m), chunks = ((pos0 + m + 15) / 16 + 31) / 32, items = sub * chunks;
     auto up = [](size_t v) { return (v + 255) / 256 * 256; };
@@ -2097,15 +2101,18 @@ static int prefill_attn_run(OmegaGpuDecodeAttnCache *c, uint32_t layer, uint32_t
     a.eps = eps;
     a.part = static_cast<float *>(cx->scratch);
     a.out_scale = out_scale;
+    const bool over = qkv_dev < out_dev + (size_t)m * 4096 && out_dev < qkv_dev + (size_t)m * 5120;
+    const uint32_t sub = over ? kPattnSubOver : kPattnSub;
     uint32_t total_items = 0, widest = 0;
     OMEGA_HIP(F_DATTN, hipEventRecord(cx->ev0, cx->stream));
-    for (uint32_t t0 = 0; t0 < m; t0 += kPattnSub) {
-        const uint32_t mm = std::min(kPattnSub, m - t0);
+    for (uint32_t t0 = 0; t0 < m; t0 += sub) {
+        const uint32_t mm = std::min(sub, m - t0);
+        float *out = out_dev + (size_t)t0 * 4096;
         a.qkv = qkv_dev + (size_t)t0 * 5120;
-        a.out = out_dev + (size_t)t0 * 4096;
         a.pos0 = pos0 + t0;
         a.m = mm;
         a.nch = pattn_chunks(a.pos0, mm);
+        a.out = a.nch == 1 && !over ? out : nullptr;
         const uint32_t pages = ((a.pos0 + mm - 1) >> 4) - (a.pos0 >> 4) + 1;
         const uint32_t items = (mm + kPattnTile - 1) / kPattnTile * a.nch;
         total_items += items;
@@ -2114,10 +2121,10 @@ static int prefill_attn_run(OmegaGpuDecodeAttnCache *c, uint32_t layer, uint32_t
         OMEGA_HIP(F_DATTN, hipGetLastError());
         OMEGA_LAUNCH(k_pattn, dim3(4 * items), dim3(512), 0, cx->stream, a);
         OMEGA_HIP(F_DATTN, hipGetLastError());
-        if (a.nch > 1) {  // a wavefront per (token, q head)
+        if (!a.out) {  // a wavefront per (token, q head)
             CombineItemsArgs cb;
             cb.part = a.part;
-            cb.out = a.out;
+            cb.out = out;
             cb.out_scale = out_scale;
             OMEGA_LAUNCH(k_attn_combine_rows, dim3((mm * 32 + 3) / 4), dim3(256), 0, cx->stream, cb, mm, a.nch);
             OMEGA_HIP(F_DATTN, hipGetLastError());

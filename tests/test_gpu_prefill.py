@@ -564,6 +564,25 @@ def test_prefill_attention_rows_of_a_split_call(omega, pf, n, split, same):
     c.free()
 
 
+@pytest.mark.parametrize("m,back", [(17, 0), (700, 0), (1500, 0), (700, 4096)])
+def test_prefill_attention_writes_over_its_input(omega, pf, m, back):
+    # the output rows over the q|k|v rows of the same call (from `back` values before them on): the
+    # rows of a call with a buffer of its own
+    rng = np.random.default_rng(m)
+    c = omega.DecodeAttnCache(1, omega.round_max_pos(900 + m), 1e6)
+    c.set_norms(0, np.ones(128, np.float32), np.ones(128, np.float32))
+    att = pf.PrefillAttention(c)
+    att.attend(0, 0, 900, rng.standard_normal((900, 5120)).astype(np.float32), 1e-6, 1.0)
+    qkv = rng.standard_normal((m, 5120)).astype(np.float32)
+    want = att.attend(0, 900, m, qkv, 1e-6, 0.5)[0]
+    d = dev_from(omega, np.concatenate([np.zeros(back, np.float32), qkv.reshape(-1)]))
+    att.attend_dev(0, 900, m, d.ptr.value + 4 * back, 1e-6, 0.5, d.ptr.value)
+    got = d.download(np.float32, m * 4096).reshape(m, 4096)
+    for t in range(m):  # where the keys are cut otherwise, the bf16 pairs round otherwise: 2^-17 each
+        assert rel_err(got[t], want[t]) <= 2 * 2.0 ** -17 + 4 * 2.0 ** -24, t
+    c.free()
+
+
 def test_prefill_attention_refusals(omega, pf):
     c = omega.DecodeAttnCache(1, 256, 1e6)
     att = pf.PrefillAttention(c)
